@@ -443,8 +443,12 @@ int styx_moe_get_hparams(const styx_moe *m, styx_moe_hparams *out);
  * NULL to skip the download). */
 int styx_moe_forward_token(styx_moe *m, uint32_t token, float *logits);
 /* generate_moe main loop (crates/model/examples/generate_moe.rs:44-67):
- * token-at-a-time prefill of the prompt, then n_predict greedy tokens
- * (the first from the prefill's logits), argmax on the device. */
+ * prefill of the prompt, then n_predict greedy tokens (the first from the
+ * prefill's logits), argmax on the device.  Prompts of more than 4 tokens
+ * run in batches of up to 512, the last token by itself: the K/V rows and
+ * logits of forwarding the tokens one by one, up to the rounding of f32
+ * sums.  (Token by token with time_kernels, with repinning, or when the
+ * batch workspace does not fit in HBM.) */
 int styx_moe_generate(styx_moe *m, const uint32_t *prompt, int n_prompt, int n_predict,
                       uint32_t *out_tokens, double *prefill_s, double *decode_s);
 /* Continue greedy decoding from the current state: n_steps forward passes,

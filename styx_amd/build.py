@@ -26,6 +26,7 @@ SOURCES = [
     "kernels_ref.hip",
     "attn.hip",
     "moe_block.hip",
+    "prompt.hip",
     "capi.cpp",
     "dispatch.cpp",
     "dispatch_fused.cpp",

@@ -185,6 +185,18 @@ struct styx_moe {
     hipStream_t st_copy = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     int n_past = 0;
+    // Prompt batches (prompt.hip): workspace of one batch of up to pb_t
+    // tokens, allocated at the first prompt long enough and kept with the
+    // model; pb_t < 0: it did not fit, prompts then run token by token.
+    int pb_t = 0;
+    struct PromptWs {
+        uint32_t *tok;
+        float *x, *xn, *q, *k, *v, *attn, *logits, *wts, *g, *u, *y, *sh_y, *gate;
+        int32_t *ids, *order, *inv;
+        int4 *tiles;
+        int *ntiles;
+        void *vec_h, *vec_o, *vec_f;  // pieces of H-, q_dim- and F-wide rows
+    } pb{};
     uint64_t repin_swaps = 0;
     std::vector<void *> dev_allocs, host_allocs;
     // timing
@@ -211,6 +223,8 @@ struct styx_moe {
     int place_experts(const std::vector<std::vector<std::pair<uint32_t, uint64_t>>> *hist);
     int enqueue_token(bool gen, int attn_mode);
     int run_token(bool gen);
+    int prompt_workspace();
+    int prompt_batch(const uint32_t *tok, int n);
     bool attn_merge_in_kernel(int n_t) const;
     int attn_mode(int n_t) const;
     int ensure_pages(int upto_pos);
@@ -983,6 +997,233 @@ int styx_moe::run_token(bool gen)
         return STYX_OK;
     }
     return enqueue_token(gen, mode);
+}
+
+// ------------------------------------------------------------- prompts ----
+// Prompts shorter than this run token by token: a batch of few tokens meets
+// nearly as many experts as its tokens do one after another, and pays about
+// twelve launches per layer instead of three.
+constexpr int PROMPT_MIN_T = 4;
+
+// The batch's workspace in one allocation; no error when it does not fit.
+int styx_moe::prompt_workspace()
+{
+    if (pb_t) return STYX_OK;
+    const int T = std::min(PROMPT_MAX_T, n_ctx);
+    const size_t qd = (size_t)nh * hd, kvd = (size_t)nkv * hd, P = (size_t)T * K;
+    const size_t fw = std::max(P * F, (size_t)T * Fsh);  // gate / up rows
+    size_t n = 0;
+    auto put = [&](auto **p, size_t bytes) {
+        *p = reinterpret_cast<std::remove_reference_t<decltype(*p)>>(n);
+        n += (bytes + 255) / 256 * 256;
+    };
+    auto lay = [&](PromptWs &w) {
+        n = 0;
+        put(&w.tok, 4 * (size_t)T);
+        put(&w.x, 4 * (size_t)T * H);
+        put(&w.xn, 4 * (size_t)T * H);
+        put(&w.q, 4 * T * qd);
+        put(&w.k, 4 * T * kvd);
+        put(&w.v, 4 * T * kvd);
+        put(&w.attn, 4 * T * qd);
+        put(&w.logits, 4 * (size_t)T * E);
+        put(&w.wts, 4 * (size_t)T * MAX_TOPK);
+        put(&w.g, 4 * fw);
+        put(&w.u, 4 * fw);
+        put(&w.y, 4 * P * H);
+        put(&w.sh_y, Fsh ? 4 * (size_t)T * H : 0);
+        put(&w.gate, 4 * (size_t)T);
+        put(&w.ids, 4 * (size_t)T * IDS_ROW);
+        put(&w.order, 4 * P);
+        put(&w.inv, 4 * P);
+        put(&w.tiles, sizeof(int4) * (P / 16 + E));
+        put(&w.ntiles, 4);
+        put((char **)&w.vec_h, prompt_vec_bytes(T, H));
+        put((char **)&w.vec_o, prompt_vec_bytes(T, (int)qd));
+        put((char **)&w.vec_f, std::max(prompt_vec_bytes(P, F), Fsh ? prompt_vec_bytes(T, Fsh) : 0));
+    };
+    lay(pb);
+    void *base = nullptr;
+    if (hipMalloc(&base, n) != hipSuccess) {
+        (void)hipGetLastError();
+        pb_t = -1;
+        return STYX_OK;
+    }
+    dev_allocs.push_back(base);
+    // the offsets laid out above become addresses
+    auto at = [&](auto **p) {
+        *p = reinterpret_cast<std::remove_reference_t<decltype(*p)>>((char *)base + (size_t)*p);
+    };
+    at(&pb.tok), at(&pb.x), at(&pb.xn), at(&pb.q), at(&pb.k), at(&pb.v), at(&pb.attn);
+    at(&pb.logits), at(&pb.wts), at(&pb.g), at(&pb.u), at(&pb.y), at(&pb.sh_y), at(&pb.gate);
+    at(&pb.ids), at(&pb.order), at(&pb.inv), at(&pb.tiles), at(&pb.ntiles);
+    at((char **)&pb.vec_h), at((char **)&pb.vec_o), at((char **)&pb.vec_f);
+    pb_t = T;
+    return STYX_OK;
+}
+
+// K and V rows of n tokens at positions n_past .. n_past + n - 1, which is
+// all that the tokens after them read: the last layer ends with its K/V rows
+// and the LM head does not run.  Enqueued only; n_past advances.
+int styx_moe::prompt_batch(const uint32_t *tok, int n)
+{
+    hipStream_t st = gpu->stream;
+    const int qd = nh * hd, kvd = nkv * hd;
+    if (int r = ensure_pages(n_past + n - 1)) return r;
+    while (n > 0) {
+        const int T = std::min(n, pb_t), P = T * K;
+        const PromptVec vh = prompt_vec_at(pb.vec_h, T, H), vo = prompt_vec_at(pb.vec_o, T, qd),
+                        vf = prompt_vec_at(pb.vec_f, P, F);
+        // positions per tile: dense matrices, and the tokens that one expert
+        // meets on average with some room above it
+        const int td = T <= 16 ? 16 : 32, te = P <= 12 * E ? 16 : 32;
+        CK(hipMemcpyAsync(pb.tok, tok, 4 * (size_t)T, hipMemcpyHostToDevice, st));
+        CK(launch_prompt_embed(st, embd.type, embd.dev, V, H, pb.tok, T, pb.x));
+        auto pack = [&](int mode, float *src, const PromptVec &v, int rows, auto fill) {
+            PromptPack p{};
+            p.src = src;
+            p.n = v.n;
+            p.eps = eps;
+            p.v = v;
+            fill(p);
+            return launch_prompt_pack(st, mode, p, rows);
+        };
+        auto dense = [&](const PromptVec &x, std::initializer_list<std::pair<const Mat *, float *>> ms, int add) {
+            // one launch per run of matrices of one type
+            PromptGemm g{};
+            g.x = x;
+            g.T = T;
+            g.add = add;
+            g.tile_tokens = td;
+            int type = -1;
+            for (auto &m : ms) {
+                if (g.nseg && m.first->type != type) {
+                    if (hipError_t e = launch_prompt_gemm(st, type, g)) return e;
+                    g.nseg = 0;
+                }
+                type = m.first->type;
+                g.w[g.nseg] = m.first->dev;
+                g.rows[g.nseg] = m.first->rows;
+                g.y[g.nseg++] = m.second;
+            }
+            return launch_prompt_gemm(st, type, g);
+        };
+        CK(pack(PACK_NORM, pb.x, vh, T, [&](PromptPack &p) { p.norm_w = layers[0].attn_norm; }));
+        for (int l = 0; l < L; l++) {
+            const Layer &ly = layers[l];
+            const bool last = l + 1 == L;
+            if (last)
+                CK(dense(vh, {{&ly.wk, pb.k}, {&ly.wv, pb.v}}, 0));
+            else
+                CK(dense(vh, {{&ly.wq, pb.q}, {&ly.wk, pb.k}, {&ly.wv, pb.v}}, 0));
+            PromptAttn a{};
+            a.q = last ? nullptr : pb.q;
+            a.k = pb.k;
+            a.v = pb.v;
+            a.q_norm = ly.q_norm;
+            a.k_norm = ly.k_norm;
+            a.eps = eps;
+            a.rope = (const double2 *)rope;
+            a.kpool = kpool;
+            a.vpool = vpool;
+            a.page_table = d_pt + (size_t)l * pages_per_layer;
+            a.page_tokens = KV_PAGE_TOKENS;
+            a.T = T;
+            a.pos0 = n_past;
+            a.nh = nh;
+            a.nkv = nkv;
+            a.hd = hd;
+            a.scale = 1.0f / std::sqrt((float)hd);
+            a.out = pb.attn;
+            CK(launch_prompt_rope(st, a));
+            if (last) break;
+            CK(launch_prompt_attn(st, a));
+            CK(pack(PACK_PLAIN, pb.attn, vo, T, [](PromptPack &) {}));
+            CK(dense(vo, {{&ly.wo, pb.x}}, 1));
+            const bool sh = ly.gsh.dev != nullptr;
+            CK(pack(PACK_NORM, pb.x, vh, T, [&](PromptPack &p) {
+                p.norm_w = ly.ffn_norm;
+                p.xn = pb.xn;
+                if (sh) {
+                    p.gate_w = ly.gate_inp_sh;
+                    p.gate_out = pb.gate;
+                }
+            }));
+            PromptRoute rt{};
+            rt.xn = pb.xn;
+            rt.W = ly.router;
+            rt.bias = ly.router_bias;
+            rt.logits = pb.logits;
+            rt.wts = pb.wts;
+            rt.ids = pb.ids;
+            rt.order = pb.order;
+            rt.inv = pb.inv;
+            rt.tiles = pb.tiles;
+            rt.ntiles = pb.ntiles;
+            rt.T = T;
+            rt.E = E;
+            rt.H = H;
+            rt.k = K;
+            rt.renorm = norm_topk;
+            rt.tile_tokens = te;
+            CK(launch_prompt_route(st, rt));
+            if (sh) {
+                const PromptVec vs = prompt_vec_at(pb.vec_f, T, Fsh);
+                CK(dense(vh, {{&ly.gsh, pb.g}, {&ly.ush, pb.u}}, 0));
+                CK(pack(PACK_SWIGLU, pb.g, vs, T, [&](PromptPack &p) { p.u = pb.u; }));
+                CK(dense(vs, {{&ly.dsh, pb.sh_y}}, 0));
+            }
+            auto experts = [&](const PromptVec &x, std::initializer_list<std::pair<const Mat *, float *>> ms,
+                               const int *order) {
+                PromptGemm g{};
+                g.x = x;
+                g.T = P;
+                g.tile_tokens = te;
+                g.tiles = pb.tiles;
+                g.ntiles = pb.ntiles;
+                // at most one tile per expert that is not full
+                g.max_tiles = std::min(P, P / te + std::min(E, P));
+                g.remap = ly.host_experts ? ly.remap_dev : nullptr;
+                g.order = order;
+                g.xdiv = K;
+                int type = -1;
+                for (auto &m : ms) {
+                    if (g.nseg && m.first->type != type) {
+                        if (hipError_t e = launch_prompt_gemm(st, type, g)) return e;
+                        g.nseg = 0;
+                    }
+                    type = m.first->type;
+                    ExpSrc &s = g.src[g.nseg];
+                    s = ExpSrc{};
+                    s.hot = ly.host_experts ? m.first->hot : m.first->dev;
+                    s.hot_slab = m.first->slab;
+                    s.gtt = m.first->host_dev;
+                    s.gtt_slab = m.first->slab;
+                    g.rows[g.nseg] = m.first->rows;
+                    g.y[g.nseg++] = m.second;
+                }
+                return launch_prompt_gemm(st, type, g);
+            };
+            CK(experts(vh, {{&ly.gate, pb.g}, {&ly.up, pb.u}}, pb.order));
+            CK(pack(PACK_SWIGLU, pb.g, vf, P, [&](PromptPack &p) { p.u = pb.u; }));
+            CK(experts(vf, {{&ly.down, pb.y}}, nullptr));
+            CK(pack(PACK_COMBINE, pb.x, vh, T, [&](PromptPack &p) {
+                p.norm_w = layers[l + 1].attn_norm;
+                p.y = pb.y;
+                p.wts = pb.wts;
+                p.inv = pb.inv;
+                p.k = K;
+                if (sh) {
+                    p.y_sh = pb.sh_y;
+                    p.gate = pb.gate;
+                }
+            }));
+        }
+        n_past += T;
+        tok += T;
+        n -= T;
+    }
+    return STYX_OK;
 }
 
 // Repin choice for one layer (moe.rs:1465-1497): residents ranked coldest
@@ -1894,7 +2135,23 @@ int styx_moe_generate(styx_moe *m, const uint32_t *prompt, int n_prompt, int n_p
         return fail(STYX_E_STATE, "prompt + generation exceeds n_ctx");
     using clk = std::chrono::steady_clock;
     const auto t0 = clk::now();
-    for (int i = 0; i < n_prompt; i++)
+    // every token but the last in batches, unless the host works between
+    // tokens (repinning counts each token's experts, timing each launch) or
+    // a token is out of range: forward_token reports that one, after the
+    // tokens before it as ever
+    int i = 0;
+    if (n_prompt > PROMPT_MIN_T && m->broken.empty() && !m->opts.time_kernels &&
+        !(m->opts.repin_interval > 0 && m->any_host)) {
+        int nb = 0;
+        while (nb < n_prompt - 1 && prompt[nb] < (uint32_t)m->V) nb++;
+        STYX_HIP(hipSetDevice(m->gpu->device));
+        if (int r = m->prompt_workspace()) return r;
+        if (m->pb_t > 0 && nb >= PROMPT_MIN_T) {
+            if (int r = m->prompt_batch(prompt, nb)) return r;
+            i = nb;
+        }
+    }
+    for (; i < n_prompt; i++)
         if (int r = styx_moe_forward_token(m, prompt[i], nullptr)) return r;
     const auto t1 = clk::now();
     // the first generated token is the prefill's argmax, already on device

@@ -309,4 +309,107 @@ hipError_t launch_clamp_copy_u32(hipStream_t st, const uint32_t *src, uint32_t *
 hipError_t launch_read_probe(hipStream_t st, const void *p, int64_t bytes, uint32_t *out,
                              int grid);
 
+// ---- prompt batches (prompt.hip) -------------------------------------------
+constexpr int PROMPT_MAX_T = 512;  // most tokens of one batch
+
+// Activation rows as three f16 pieces of x 2^e, [3][rows][np] (np: n rounded
+// up to whole 256-value steps, zeros past n), the sums of each run of 32
+// values as pieces of sum 2^(e-6), [rows][np/256][4][8] (the fourth piece
+// zero), and 2^-e per row.
+struct PromptVec {
+    uint16_t *p, *sums;
+    float *scale;
+    int n, np;
+    int64_t rows;
+};
+inline int prompt_np(int n) { return (n + 255) / 256 * 256; }
+inline size_t prompt_vec_bytes(int64_t rows, int n)
+{
+    const size_t np = (size_t)prompt_np(n), r = (size_t)((rows + 63) / 64 * 64);
+    return 3 * r * np * 2 + r * (np / 256) * 64 + r * 4;
+}
+inline PromptVec prompt_vec_at(void *base, int64_t rows, int n)
+{
+    const int64_t r = (rows + 63) / 64 * 64;
+    PromptVec v;
+    v.n = n;
+    v.np = prompt_np(n);
+    v.rows = r;
+    v.p = (uint16_t *)base;
+    v.sums = v.p + 3 * r * v.np;
+    v.scale = (float *)(v.sums + r * (v.np / 256) * 32);
+    return v;
+}
+
+enum PackMode { PACK_PLAIN = 0, PACK_NORM, PACK_SWIGLU, PACK_COMBINE };
+struct PromptPack {
+    float *src;           // [rows][n] (PACK_COMBINE: the residual, updated)
+    const float *u;       // PACK_SWIGLU: [rows][n]
+    int n;
+    const float *norm_w;  // PACK_NORM, PACK_COMBINE
+    float eps;
+    float *xn;            // optional: the normalised rows
+    const float *gate_w;  // optional: gate_out[row] = gate_w . normalised row
+    float *gate_out;
+    const float *y;       // PACK_COMBINE: [places][n], weights [rows][MAX_TOPK]
+    const float *wts;
+    const int *inv;       // place of pair row k + s, or -1
+    int k;
+    const float *y_sh, *gate;  // optional: sigmoid(gate[row]) y_sh[row] added
+    PromptVec v;
+};
+
+// Rows of up to 3 matrices of one type times activation rows: dense
+// (positions 0..T) or, with tiles, the positions of each tile's expert.
+struct PromptGemm {
+    PromptVec x;
+    int T;                 // dense: positions
+    const uint8_t *w[3];
+    int rows[3];
+    float *y[3];           // [positions][rows]
+    int nseg, add;
+    int tile_tokens;       // 16 or 32 positions per workgroup
+    const int4 *tiles;     // {expert, first position, positions, 0}
+    const int *ntiles;
+    int max_tiles;
+    ExpSrc src[3];         // per segment, with tiles
+    const uint32_t *remap; // expert -> hot slot or SKIP (read from gtt); null: itself
+    const int *order;      // activation row of a position: order[pos] / xdiv; null: pos
+    int xdiv;
+    int rt0[3], nrt, ntt;  // filled by the launch
+};
+
+struct PromptAttn {
+    float *q;              // [T][nh*hd]; rope: rotated in place (null: K/V only)
+    const float *k, *v;    // [T][nkv*hd] raw projections
+    const float *q_norm, *k_norm;
+    float eps;
+    const double2 *rope;   // [n_pos][hd/2]
+    float *kpool, *vpool;  // [pages][nkv][page_tokens][hd]
+    const int32_t *page_table;
+    int page_tokens, T, pos0, nh, nkv, hd;
+    float scale;
+    float *out;            // [T][nh*hd]
+};
+
+struct PromptRoute {
+    const float *xn, *W, *bias;
+    float *logits;         // [T][E]
+    float *wts;            // [T][MAX_TOPK]
+    int32_t *ids;          // [T][IDS_ROW]
+    int *order, *inv;      // [T*k]
+    int4 *tiles;
+    int *ntiles;
+    int T, E, H, k, renorm, tile_tokens;
+};
+
+hipError_t launch_prompt_embed(hipStream_t st, int t, const uint8_t *w, int64_t nrows, int ncols,
+                               const uint32_t *tok, int T, float *x);
+hipError_t launch_prompt_pack(hipStream_t st, int mode, const PromptPack &a, int rows);
+hipError_t launch_prompt_gemm(hipStream_t st, int t, PromptGemm a);
+hipError_t launch_prompt_rope(hipStream_t st, const PromptAttn &a);
+hipError_t launch_prompt_attn(hipStream_t st, const PromptAttn &a);
+// Router logits, top-k ids and weights, and the pairs grouped by expert.
+hipError_t launch_prompt_route(hipStream_t st, const PromptRoute &a);
+
 }  // namespace styx
