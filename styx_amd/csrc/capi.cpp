@@ -58,6 +58,7 @@ static void gpu_destroy(styx_gpu *g)
     hipStreamDestroy(g->stream);
     if (g->xq_scratch) hipFree(g->xq_scratch);
     if (g->partial_scratch) hipFree(g->partial_scratch);
+    if (g->ref_part) hipFree(g->ref_part);
     if (g->fused_scalars) hipFree(g->fused_scalars);
     if (g->fused_pt) hipFree(g->fused_pt);
     delete g;
@@ -113,6 +114,7 @@ int styx_gpu_new(int device, styx_gpu **out)
     if (e != hipSuccess) {
         if (g->xq_scratch) hipFree(g->xq_scratch);
         if (g->partial_scratch) hipFree(g->partial_scratch);
+    if (g->ref_part) hipFree(g->ref_part);
         if (g->fused_scalars) hipFree(g->fused_scalars);
         if (g->fused_pt) hipFree(g->fused_pt);
         hipStreamDestroy(g->stream);

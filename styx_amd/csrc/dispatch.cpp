@@ -32,6 +32,7 @@ struct styx_batch {
     hipStream_t own = nullptr;
     hipEvent_t done = nullptr;
     bool pending = false;
+    float *part = nullptr;  // an async batch's own attention partials
     struct Cmd {
         const styx_kernel *k;
         std::vector<void *> ptr;
@@ -99,16 +100,35 @@ struct styx_timeline {
 
 namespace {
 
+// Attention partials for work on b's stream: the batch's own when it has a
+// stream of its own, else the gpu's (its caller holds ref_mu).  Without
+// memory for them contexts are not split.
+RefScratch ref_scratch(styx_batch *b)
+{
+    float *&p = b->own ? b->part : b->gpu->ref_part;
+    if (!p && hipMalloc((void **)&p, REF_SCRATCH_FLOATS * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+    return RefScratch{p, REF_SCRATCH_FLOATS};
+}
+
 // The recorded work of b, launched in order on stream st.
 int run_cmds(styx_batch *b, hipStream_t st)
 {
     for (auto &c : b->cmds) {
+        std::unique_lock<std::mutex> lock;
+        RefScratch scratch{};
+        if (c.k->kid == RK_ATTN) {
+            if (!b->own) lock = std::unique_lock<std::mutex>(b->gpu->ref_mu);
+            scratch = ref_scratch(b);
+        }
         const uint32_t *spec = c.k->spec.empty() ? nullptr : c.k->spec.data();
         hipError_t e = c.k->kid >= RK_F_ROUTER_TOPK
                            ? fused_launch(b->gpu, st, c.k->kid, c.ptr.data(), c.size.data(),
                                           c.push.data())
                            : refk_launch(st, c.k->kid, c.ptr.data(), c.size.data(), c.push.data(),
-                                         c.gx, c.gy, c.gz, spec, (int)c.k->spec.size() / 2);
+                                         c.gx, c.gy, c.gz, spec, (int)c.k->spec.size() / 2, &scratch);
         if (e == hipErrorInvalidValue)
             return fail(STYX_E_INVALID, c.k->name + ": unsupported parameters, or the push "
                                                     "constants and grid reach past a binding");
@@ -232,6 +252,7 @@ void styx_batch_free(styx_batch *b)
         hipStreamSynchronize(b->own);
         hipEventDestroy(b->done);
         hipStreamDestroy(b->own);
+        if (b->part) hipFree(b->part);
     }
     delete b;
     gpu_release(g);

@@ -3,7 +3,7 @@
 // bindings and push-constant block of the shader or vendored kernel it
 // stands in for, with the same workgroup grid.  Quant weights are read in
 // GGUF block layout, as the reference uploads them.
-#include "deq.h"
+#include "attn16.h"
 #include "kernels.h"
 #include "qdot.h"
 #include "refk.h"
@@ -44,25 +44,46 @@ __global__ void __launch_bounds__(256) kr_axpy_sig(const float *a, const float *
     if (i < n) d[i] += s * a[i];
 }
 
-// shaders/matvec_strided_f32.comp: 32 strided partials, halving tree.
-__global__ void __launch_bounds__(32) kr_matvec_strided(const float *A, const float *x, float *d,
+#pragma clang fp contract(on)
+
+// shaders/matvec_strided_f32.comp: one row per wave.  A router row is a few
+// KB and a launch has few rows, so a row's time is its memory round trip:
+// every lane has its loads of a 2048-value pass (8 of the row, 8 of x) in
+// flight at once.  128 rows of 2048: 21.6 us with 32 lanes and one load at a
+// time, 4.9 so.
+__global__ void __launch_bounds__(64) kr_matvec_strided(const float *A, const float *x, float *d,
                                                         uint32_t ncols, uint32_t stride)
 {
-    __shared__ float tmp[32];
     const uint32_t row = blockIdx.x, tid = threadIdx.x;
     const float *a = A + (int64_t)row * stride;
     float sum = 0.0f;
-    for (uint32_t c = tid; c < ncols; c += 32) sum += a[c] * x[c];
-    tmp[tid] = sum;
-    __syncthreads();
-    for (uint32_t s = 16; s > 0; s >>= 1) {
-        if (tid < s) tmp[tid] += tmp[tid + s];
-        __syncthreads();
+    uint32_t c0 = 0;
+    for (; c0 + 2048 <= ncols; c0 += 2048) {
+        f4 av[8], xv[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            av[j] = ld4(a + c0 + 256 * j + 4 * tid);
+            xv[j] = ld4(x + c0 + 256 * j + 4 * tid);
+        }
+        float p[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            p[j] = av[j].x * xv[j].x + av[j].y * xv[j].y + av[j].z * xv[j].z + av[j].w * xv[j].w;
+        sum += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
     }
-    if (tid == 0) d[row] = tmp[0];
+    for (; c0 + 256 <= ncols; c0 += 256) {
+        const f4 av = ld4(a + c0 + 4 * tid), xv = ld4(x + c0 + 4 * tid);
+        sum += av.x * xv.x + av.y * xv.y + av.z * xv.z + av.w * xv.w;
+    }
+    for (uint32_t c = c0 + tid; c < ncols; c += 64) sum += a[c] * x[c];
+    sum = wave_sum(sum);
+    if (tid == 0) d[row] = sum;
 }
 
-// shaders/attn_decode_f32.comp:31-79 (one workgroup of 128 per query head).
+#pragma clang fp contract(off)
+
+// shaders/attn_decode_f32.comp:31-79 (one workgroup of 128 per query head),
+// for head dimensions without a matrix-core kernel and for empty contexts.
 __global__ void __launch_bounds__(128) kr_attn_decode(const float *Q, const float *K,
                                                       const float *V, float *O, uint32_t n_t,
                                                       uint32_t hd, uint32_t kv_dim, uint32_t gqa,
@@ -109,6 +130,102 @@ __global__ void __launch_bounds__(128) kr_attn_decode(const float *Q, const floa
     if (tid + 128 < hd) O[qbase + tid + 128] = acc1 * inv_l;
 }
 
+#pragma clang fp contract(on)
+
+// attn_decode_f32 for head dimensions 64, 128 and 256: 16 query heads of one
+// kv head per workgroup (attn16.h), so that each K/V row is read once per
+// kv head, four waves on every fourth block of 32 keys.  Bound by the keys'
+// round trips: a long context is cut into `chunk` keys per workgroup
+// (blockIdx.x) whose (m, l, o) go to part [head][chunks][hd + 2] and are
+// merged by kr_attn_merge.  Against one workgroup per query head and a
+// barrier tree per key: 145 keys 167 -> 8 us, 4000 keys 5360 -> 16 us
+// (32 heads, 4 kv heads of 128).
+struct AttnRef {
+    const float *Q, *K, *V;
+    float *O, *part;  // part: null with one chunk
+    uint32_t n_t, kv_dim, gqa, nh, tiles, chunk;  // tiles: of 16 heads per kv head
+    float scale;
+};
+
+template <int HD> __global__ void __launch_bounds__(256) kr_attn16(AttnRef a)
+{
+    __shared__ __align__(16) Merge16<HD> s;
+    const uint32_t kvh = blockIdx.y / a.tiles, h0 = kvh * a.gqa + blockIdx.y % a.tiles * 16;
+    const uint32_t nrow = min(min(a.gqa - blockIdx.y % a.tiles * 16, 16u), a.nh - min(h0, a.nh));
+    if (nrow == 0) return;
+    const uint32_t c0 = blockIdx.x * a.chunk, c1 = min(a.n_t, c0 + a.chunk);
+    Attn16<HD> at;
+    at.init(a.Q + (int64_t)(h0 + min((uint32_t)(threadIdx.x & 15), nrow - 1)) * HD);
+    for (uint32_t k0 = c0 + (threadIdx.x >> 6) * A16_KB; k0 < c1; k0 += 4 * A16_KB) {
+        const int64_t base = (int64_t)k0 * a.kv_dim + (int64_t)kvh * HD;
+        const int left = (int)min(c1 - k0, (uint32_t)A16_KB);
+        at.block(a.K + base, a.V + base, a.kv_dim, left - 1, left, a.scale);
+    }
+    attn16_merge<HD>(at, s, [&](int r, int d, float O, float L, float M) {
+        if ((uint32_t)r >= nrow) return;
+        const int64_t h = h0 + r;
+        if (!a.part) {
+            a.O[h * HD + d] = O / L;
+            return;
+        }
+        float *p = a.part + (h * gridDim.x + blockIdx.x) * (HD + 2);
+        p[2 + d] = O;
+        if (d == 0) p[0] = M, p[1] = L;
+    });
+}
+
+// One workgroup per query head, one thread per dimension: the chunks'
+// largest maximum, then their sums in order.
+__global__ void __launch_bounds__(256) kr_attn_merge(const float *part, float *O, int chunks)
+{
+    const int hd = blockDim.x, d = threadIdx.x;
+    const float *p = part + (int64_t)blockIdx.x * chunks * (hd + 2);
+    float M = -INFINITY;
+    for (int c = 0; c < chunks; c++) M = fmaxf(M, p[(int64_t)c * (hd + 2)]);
+    float L = 0.0f, o = 0.0f;
+#pragma unroll 8
+    for (int c = 0; c < chunks; c++) {
+        const float *q = p + (int64_t)c * (hd + 2);
+        const float f = q[0] == -INFINITY ? 0.0f : expf(q[0] - M);
+        L += q[1] * f;
+        o += q[2 + d] * f;
+    }
+    O[(int64_t)blockIdx.x * hd + d] = o / L;
+}
+
+// Chunks of a context of n_t keys for ny workgroups per chunk and gx heads:
+// one up to 256 keys (two blocks per wave: a merge kernel costs more), else
+// of 128 keys (one block per wave) while the launch has at most 512
+// workgroups, two per CU, and the partials fit the scratch.
+static uint32_t attn_chunk_keys(uint64_t n_t, uint64_t ny, uint64_t gx, uint64_t hd, const RefScratch *s)
+{
+    if (n_t <= 256 || !s || !s->p) return (uint32_t)n_t;
+    const uint64_t most = std::min<uint64_t>(512 / std::min<uint64_t>(ny, 512), s->floats / (gx * (hd + 2)));
+    if (most < 2) return (uint32_t)n_t;
+    return (uint32_t)std::min<uint64_t>(n_t, (n_t + 128 * most - 1) / (128 * most) * 128);
+}
+
+static hipError_t attn_go(hipStream_t st, AttnRef a, uint32_t hd, const RefScratch *s)
+{
+    a.tiles = (a.gqa + 15) / 16;
+    const uint64_t ny = (uint64_t)((a.nh + a.gqa - 1) / a.gqa) * a.tiles;
+    if (ny > 65535) return hipErrorNotSupported;
+    a.chunk = attn_chunk_keys(a.n_t, ny, a.nh, hd, s);
+    const uint32_t chunks = (a.n_t + a.chunk - 1) / a.chunk;
+    a.part = chunks > 1 ? s->p : nullptr;
+    const dim3 grid(chunks, (unsigned)ny);
+    if (hd == 64)
+        hipLaunchKernelGGL(kr_attn16<64>, grid, dim3(256), 0, st, a);
+    else if (hd == 128)
+        hipLaunchKernelGGL(kr_attn16<128>, grid, dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(kr_attn16<256>, grid, dim3(256), 0, st, a);
+    if (chunks > 1) hipLaunchKernelGGL(kr_attn_merge, dim3(a.nh), dim3(hd), 0, st, a.part, a.O, (int)chunks);
+    return hipGetLastError();
+}
+
+#pragma clang fp contract(off)
+
 // swiglu_f32 split mode over n values (GluPush.n).
 __global__ void __launch_bounds__(256) kr_swiglu(const float *g, const float *u, float *d, uint32_t n)
 {
@@ -133,8 +250,20 @@ __global__ void __launch_bounds__(256) kr_rms_norm(const float *a, const float *
 
 #pragma clang fp contract(on)
 
-// mul_mat_vec_{t} / mul_mat_vec_id_{t} over GGUF-layout rows: one wave per
-// (row, slot); lanes take blocks, dequantize in reference order and dot.
+// mul_mat_vec_{t} / mul_mat_vec_id_{t} over GGUF-layout rows.  A row is cut
+// into units of 32 values (one q8_0 block, or an eighth of a K-quant block:
+// 16 bytes of quants hold its low-nibble values and, 32 or 64 values on, its
+// high-nibble ones), so that a lane group of cols / 32 lanes reads a row's
+// blocks end to end in 16-byte loads.  A lane keeps its units' activations
+// in registers over the rows its group visits and has the next row's loads
+// in flight over this row's products, which are f32 FMAs of the integer
+// quants; the unit's factors multiply the sums.
+//
+// Bound: the memory round trip at one expert's few rows, the weight stream
+// beyond.  Against one lane per block and byte loads into a dequantized
+// array in scratch memory (8 of 64 lanes busy on a 2048-column K-quant row),
+// 30B-A3B layer: gate q4_K 183 -> 8, up q5_K 178 -> 8, down q6_K 382 -> 9,
+// q q8_0 24 -> 6 us.
 struct MmvRef {
     const uint8_t *A;
     const float *B;
@@ -142,38 +271,244 @@ struct MmvRef {
     const int32_t *ids;  // null for the plain matvec
     int type;
     uint32_t ncols, stride_a, stride_b, stride_d, batch_stride_a, batch_stride_b, batch_stride_d;
-    uint32_t ne11, expert_i1, nbi1, nrows, num_rows;
+    uint32_t ne11, expert_i1, nbi1, nrows;
     int64_t n_mat;  // matrices readable from A (ids at or past it are skipped)
+    int G;          // lanes per row (a power of two)
+    int passes;     // rows per lane group
 };
 
-__global__ void __launch_bounds__(64) kr_mmv(MmvRef p)
+constexpr int MMV_WG = 256;
+
+// 16 bytes at a 2-byte aligned address (34- and 210-byte blocks).
+__device__ __forceinline__ styx_u4 ld16u(const uint8_t *p)
 {
-    const int t = p.type, be = blk_elems(t), bb = blk_bytes(t);
+    struct __attribute__((packed, aligned(2))) U { uint32_t w[4]; };
+    const U *u = (const U *)p;
+    return styx_u4{u->w[0], u->w[1], u->w[2], u->w[3]};
+}
+__device__ __forceinline__ styx_u4 ld16(const uint8_t *p) { return *(const styx_u4 *)p; }
+
+template <int N> __device__ __forceinline__ float ubyte(uint32_t v) { return (float)((v >> (8 * N)) & 255u); }
+
+// sum of 16 unsigned bytes times x[0..16)
+__device__ __forceinline__ float dot16(const styx_u4 q, const float *x)
+{
+    float s[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        s[i] = fmaf(ubyte<0>(q[i]), x[4 * i], ubyte<1>(q[i]) * x[4 * i + 1]) +
+               fmaf(ubyte<2>(q[i]), x[4 * i + 2], ubyte<3>(q[i]) * x[4 * i + 3]);
+    return (s[0] + s[1]) + (s[2] + s[3]);
+}
+__device__ __forceinline__ float dot16s(const styx_u4 q, const float *x)  // signed bytes
+{
+    float s[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        s[i] = fmaf((float)(int8_t)q[i], x[4 * i], (float)(int8_t)(q[i] >> 8) * x[4 * i + 1]) +
+               fmaf((float)(int8_t)(q[i] >> 16), x[4 * i + 2], (float)((int32_t)q[i] >> 24) * x[4 * i + 3]);
+    return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+// One unit's activations: two runs of 16 values and their sums.
+struct MX {
+    float x[32], s0, s1;
+    __device__ __forceinline__ void load(const float *b, int lo, int hi)
+    {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const f4 u = ld4(b + lo + 4 * i), v = ld4(b + hi + 4 * i);
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[4 * i + j] = u[j], x[16 + 4 * i + j] = v[j];
+        }
+        s0 = s1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) s0 += x[i], s1 += x[16 + i];
+    }
+};
+
+// Unit u of a row: its block, the first value of its two runs, its loads
+// and its share of the dot product.
+template <int T> struct MU;
+template <> struct MU<T_Q8_0> {
+    styx_u4 q0, q1;
+    uint32_t d;
+    static __device__ __forceinline__ void runs(int u, int &lo, int &hi) { lo = 32 * u, hi = lo + 16; }
+    __device__ __forceinline__ void load(const uint8_t *row, int u)
+    {
+        const uint8_t *b = row + 34 * (int64_t)u;
+        d = *(const uint16_t *)b;
+        q0 = ld16u(b + 2);
+        q1 = ld16u(b + 18);
+    }
+    __device__ __forceinline__ float dot(const MX &x, int) const
+    {
+        return f16f(d) * (dot16s(q0, x.x) + dot16s(q1, x.x + 16));
+    }
+};
+// q4_K / q5_K: part p = u & 7 reads quant bytes [16 p, +16): run h = p & 1
+// of quarter c = p >> 1.
+template <int T> struct MUK {
+    styx_u4 q, hd, qh;
+    static __device__ __forceinline__ void runs(int u, int &lo, int &hi)
+    {
+        lo = 256 * (u >> 3) + 64 * ((u >> 1) & 3) + 16 * (u & 1);
+        hi = lo + 32;
+    }
+    __device__ __forceinline__ void load(const uint8_t *row, int u)
+    {
+        const uint8_t *b = row + (T == T_Q4_K ? 144 : 176) * (int64_t)(u >> 3);
+        hd = ld16(b);
+        q = ld16(b + (T == T_Q4_K ? 16 : 48) + 16 * (u & 7));
+        if (T == T_Q5_K) qh = ld16(b + 16 + 16 * (u & 1));
+    }
+    __device__ __forceinline__ float dot(const MX &x, int u) const
+    {
+        const int c = (u >> 1) & 3;
+        styx_u4 lo = q & 0x0F0F0F0Fu, hi = (q >> 4) & 0x0F0F0F0Fu;
+        if (T == T_Q5_K) {
+            const styx_u4 h = qh >> (uint32_t)(2 * c);
+            lo |= (h & 0x01010101u) << 4;
+            hi |= (h & 0x02020202u) << 3;
+        }
+        float s0, s1, m0, m1;
+        k4_scales(make_uint4(hd.x, hd.y, hd.z, hd.w), 16 * (c & 1), c >> 1, s0, s1, m0, m1);
+        const float d = f16f(hd.x), dm = f16f(hd.x >> 16);
+        return ((d * s0) * dot16(lo, x.x) - (dm * m0) * x.s0) +
+               ((d * s1) * dot16(hi, x.x + 16) - (dm * m1) * x.s1);
+    }
+};
+template <> struct MU<T_Q4_K> : MUK<T_Q4_K> {};
+template <> struct MU<T_Q5_K> : MUK<T_Q5_K> {};
+// q6_K: part p = u & 7 reads low bits [16 p, +16): half n = p >> 2, run
+// j = (p >> 1) & 1, piece h = p & 1.
+template <> struct MU<T_Q6_K> {
+    styx_u4 q, qh;
+    uint32_t sc, d;  // the two runs' scales, bytes 0 and 2
+    static __device__ __forceinline__ void runs(int u, int &lo, int &hi)
+    {
+        const int p = u & 7;
+        lo = 256 * (u >> 3) + 128 * (p >> 2) + 32 * ((p >> 1) & 1) + 16 * (p & 1);
+        hi = lo + 64;
+    }
+    __device__ __forceinline__ void load(const uint8_t *row, int u)
+    {
+        const int p = u & 7, n = p >> 2;
+        const uint8_t *b = row + 210 * (int64_t)(u >> 3);
+        q = ld16u(b + 16 * p);
+        qh = ld16u(b + 128 + 32 * n + 16 * (p & 1));
+        const uint8_t *s = b + 192 + 8 * n + (p & 3);
+        sc = (uint32_t)s[0] | (uint32_t)s[4] << 16;
+        d = *(const uint16_t *)(b + 208);
+    }
+    __device__ __forceinline__ float dot(const MX &x, int u) const
+    {
+        const uint32_t j2 = 2 * ((u >> 1) & 1);
+        const styx_u4 lo = (q & 0x0F0F0F0Fu) | (((qh >> j2) & 0x03030303u) << 4);
+        const styx_u4 hi = ((q >> 4) & 0x0F0F0F0Fu) | (((qh >> (j2 + 4u)) & 0x03030303u) << 4);
+        const float s0 = (float)(int8_t)sc, s1 = (float)(int8_t)(sc >> 16);
+        return f16f(d) * (s0 * (dot16(lo, x.x) - 32.0f * x.s0) + s1 * (dot16(hi, x.x + 16) - 32.0f * x.s1));
+    }
+};
+
+// UPL: units per lane whose activations stay in registers (1 or 2; rows of
+// up to 64 or 128 units); 0: any length, activations read again per row.
+template <int T, int UPL> __global__ void __launch_bounds__(MMV_WG) kr_mmv(MmvRef p)
+{
+    constexpr int bb = T == T_Q8_0 ? 34 : T == T_Q4_K ? 144 : T == T_Q5_K ? 176 : 210;
+    constexpr int be = T == T_Q8_0 ? 32 : 256;
     const uint32_t slot = blockIdx.y;
-    int64_t a_blk = 0, b_off = 0, d_off = 0;
+    const uint8_t *A = p.A;
+    int64_t b_off = 0, d_off = 0;
     if (p.ids) {
         // get_offsets() of mul_mat_vec_base (crates/vk-backend/tests/kernels.rs:124-131)
         const uint32_t e = (uint32_t)p.ids[slot + p.expert_i1 * p.nbi1];
         if (e == SKIP || (int64_t)e >= p.n_mat) return;
-        a_blk = (int64_t)e * (p.batch_stride_a / be);
+        A += (int64_t)e * (p.batch_stride_a / be) * bb;
         b_off = (int64_t)(slot % p.ne11) * p.stride_b + (int64_t)p.expert_i1 * p.batch_stride_b;
         d_off = (int64_t)slot * p.stride_d + (int64_t)p.expert_i1 * p.batch_stride_d;
     }
-    const uint32_t nb = p.ncols / be;
-    for (uint32_t j = 0; j < p.num_rows; j++) {
-        const uint32_t r = blockIdx.x * p.num_rows + j;
-        if (r >= p.nrows) return;
-        float acc = 0.0f;
-        for (uint32_t b = threadIdx.x; b < nb; b += 64) {
-            const uint8_t *blk = p.A + (a_blk + (int64_t)r * p.stride_a + b) * bb;
-            float y[256];
-            deq_block(t, gguf_blk(blk, t), 0, y, false);
-            const float *x = p.B + b_off + (int64_t)b * be;
-            for (int i = 0; i < be; i++) acc += y[i] * x[i];
+    const int lg = __builtin_ctz((unsigned)p.G);
+    const int lane = threadIdx.x & 63, gl = lane & (p.G - 1), ngrp = MMV_WG >> lg;
+    const int64_t first = (int64_t)blockIdx.x * ngrp * p.passes + (threadIdx.x >> lg);
+    const int nu = (int)(p.ncols / 32);
+    const float *B = p.B + b_off;
+    const int64_t rb = (int64_t)p.stride_a * bb;
+    auto row_at = [&](int i) {
+        return A + rb * min(first + (int64_t)i * ngrp, (int64_t)p.nrows - 1);
+    };
+    auto put = [&](int i, float v) {
+        v = group_sum(v, gl, p.G);
+        const int64_t r = first + (int64_t)i * ngrp;
+        if (gl == 0 && r < p.nrows) p.D[d_off + r] = v;
+    };
+    if constexpr (UPL > 0) {
+        MX x[UPL];
+        MU<T> w[UPL];
+        // a lane past the row's units works on unit 0 and adds nothing
+        int un[UPL];
+        bool on[UPL];
+#pragma unroll
+        for (int j = 0; j < UPL; j++) {
+            on[j] = gl + j * p.G < nu;
+            un[j] = on[j] ? gl + j * p.G : 0;
+            w[j].load(row_at(0), un[j]);
         }
-        acc = wave_sum(acc);
-        if (threadIdx.x == 0) p.D[d_off + r] = acc;
+#pragma unroll
+        for (int j = 0; j < UPL; j++) {
+            int lo, hi;
+            MU<T>::runs(un[j], lo, hi);
+            x[j].load(B, lo, hi);
+        }
+        for (int i = 0; i < p.passes; i++) {
+            MU<T> c[UPL];
+#pragma unroll
+            for (int j = 0; j < UPL; j++) {
+                c[j] = w[j];
+                if (i + 1 < p.passes) w[j].load(row_at(i + 1), un[j]);
+            }
+            float v = 0.0f;
+#pragma unroll
+            for (int j = 0; j < UPL; j++) {
+                const float t = c[j].dot(x[j], un[j]);
+                if (on[j]) v += t;
+            }
+            put(i, v);
+        }
+    } else {
+        for (int i = 0; i < p.passes; i++) {
+            const uint8_t *row = row_at(i);
+            float v = 0.0f;
+            for (int u = gl; u < nu; u += p.G) {
+                MU<T> w;
+                MX x;
+                int lo, hi;
+                w.load(row, u);
+                MU<T>::runs(u, lo, hi);
+                x.load(B, lo, hi);
+                v += w.dot(x, u);
+            }
+            put(i, v);
+        }
     }
+}
+
+template <int T> static void mmv_go(hipStream_t st, MmvRef &p, uint32_t slots)
+{
+    const uint32_t nu = p.ncols / 32;
+    p.G = 1;
+    while (p.G < 64 && (uint32_t)p.G < nu) p.G *= 2;
+    // about 4096 waves over all slots' rows, at least one row per lane group
+    const uint64_t ngrp = MMV_WG / p.G, groups = 4096ull * 64 / p.G;
+    p.passes = (int)std::max<uint64_t>(1, ((uint64_t)p.nrows * slots + groups - 1) / groups);
+    const uint64_t per = ngrp * p.passes;
+    const dim3 grid((unsigned)((p.nrows + per - 1) / per), slots);
+    if (nu <= 64)
+        hipLaunchKernelGGL((kr_mmv<T, 1>), grid, dim3(MMV_WG), 0, st, p);
+    else if (nu <= 128)
+        hipLaunchKernelGGL((kr_mmv<T, 2>), grid, dim3(MMV_WG), 0, st, p);
+    else
+        hipLaunchKernelGGL((kr_mmv<T, 0>), grid, dim3(MMV_WG), 0, st, p);
 }
 
 // topk_softmax_f32 with the shader's bindings (remap/pmap required).
@@ -260,7 +595,7 @@ static bool fits(uint64_t size, uint64_t n, uint64_t bytes_each)
 
 hipError_t refk_launch(hipStream_t st, int kid, void *const *ptr, const uint64_t *size,
                        const void *push, uint32_t gx, uint32_t gy, uint32_t gz,
-                       const uint32_t *spec, int n_spec)
+                       const uint32_t *spec, int n_spec, const RefScratch *scratch)
 {
     const uint32_t *pc = (const uint32_t *)push;
     const hipError_t bad = hipErrorInvalidValue;
@@ -289,7 +624,7 @@ hipError_t refk_launch(hipStream_t st, int kid, void *const *ptr, const uint64_t
         if (!fits(size[0], (uint64_t)(gx - 1) * stride + nc, 4) || !fits(size[1], nc, 4) ||
             !fits(size[2], gx, 4))
             return bad;
-        hipLaunchKernelGGL(kr_matvec_strided, dim3(gx), dim3(32), 0, st, (const float *)ptr[0],
+        hipLaunchKernelGGL(kr_matvec_strided, dim3(gx), dim3(64), 0, st, (const float *)ptr[0],
                            (const float *)ptr[1], (float *)ptr[2], pc[0], pc[1]);
         break;
     }
@@ -303,6 +638,20 @@ hipError_t refk_launch(hipStream_t st, int kid, void *const *ptr, const uint64_t
         if (!fits(size[0], (uint64_t)gx * hd, 4) || !fits(size[1], kv_need, 4) ||
             !fits(size[2], kv_need, 4) || !fits(size[3], (uint64_t)gx * hd, 4))
             return bad;
+        if (n_t > 0 && (hd == 64 || hd == 128 || hd == 256)) {
+            AttnRef a{};
+            a.Q = (const float *)ptr[0];
+            a.K = (const float *)ptr[1];
+            a.V = (const float *)ptr[2];
+            a.O = (float *)ptr[3];
+            a.n_t = pc[0];
+            a.kv_dim = pc[2];
+            a.gqa = (uint32_t)std::min<uint64_t>(gqa, gx);
+            a.nh = gx;
+            a.scale = scale;
+            const hipError_t e = attn_go(st, a, pc[1], scratch);
+            if (e != hipErrorNotSupported) return e;
+        }
         hipLaunchKernelGGL(kr_attn_decode, dim3(gx), dim3(128), 0, st, (const float *)ptr[0],
                            (const float *)ptr[1], (const float *)ptr[2], (float *)ptr[3], pc[0],
                            pc[1], pc[2], pc[3], scale);
@@ -445,7 +794,6 @@ hipError_t refk_launch(hipStream_t st, int kid, void *const *ptr, const uint64_t
             p.expert_i1 = pc[10];
             p.nbi1 = pc[11];
             p.nrows = gx;
-            p.num_rows = 1;
             if (p.batch_stride_a % be) return bad;
             // one matrix: nrows rows of stride_a blocks, within the expert stride
             const uint64_t mat_blocks = (uint64_t)p.batch_stride_a / be;
@@ -462,16 +810,24 @@ hipError_t refk_launch(hipStream_t st, int kid, void *const *ptr, const uint64_t
                 return bad;
         } else {
             // MatVecPush: stride_d = nrows (MatVecPush::simple); NUM_ROWS spec id 1
-            p.num_rows = 1;
+            uint64_t num_rows = 1;
             for (int i = 0; i + 1 < 2 * n_spec; i += 2)
-                if (spec[i] == 1) p.num_rows = spec[i + 1] ? spec[i + 1] : 1;
+                if (spec[i] == 1) num_rows = spec[i + 1] ? spec[i + 1] : 1;
             p.nrows = p.stride_d;
             p.n_mat = 1;
             if (p.nrows == 0 || !fits(size[0], (uint64_t)(p.nrows - 1) * p.stride_a + nb, bb) ||
                 !fits(size[1], p.ncols, 4) || !fits(size[2], p.nrows, 4))
                 return bad;
+            // the rows the grid covers
+            p.nrows = (uint32_t)std::min<uint64_t>(p.nrows, num_rows * gx);
         }
-        hipLaunchKernelGGL(kr_mmv, dim3(gx, with_id ? gy : 1, 1), dim3(64), 0, st, p);
+        const uint32_t slots = with_id ? gy : 1;
+        switch (p.type) {
+        case T_Q8_0: mmv_go<T_Q8_0>(st, p, slots); break;
+        case T_Q4_K: mmv_go<T_Q4_K>(st, p, slots); break;
+        case T_Q5_K: mmv_go<T_Q5_K>(st, p, slots); break;
+        default: mmv_go<T_Q6_K>(st, p, slots); break;
+        }
         break;
     }
     }

@@ -30,6 +30,7 @@
 // bits were dropped downwards by the matrix core, an error of one sign
 // (-0.3 ulp on average over q8_0 rows) that attention over many keys does
 // not average out.
+#include "attn16.h"
 #include "deq.h"
 #include "head.h"
 #include "kernels.h"
@@ -42,7 +43,6 @@ namespace styx {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int PWG = 256;                 // threads of every kernel here but the plan
 constexpr int KC = 256;                  // values of a row per GEMM step
@@ -732,141 +732,34 @@ template <int PPL> __global__ void __launch_bounds__(PWG) k_prompt_rope(PromptAt
 // ------------------------------------------------------------ attention ----
 // Causal attention of T tokens at positions pos0.. over cached keys: a
 // workgroup takes 16 query rows (token, head) of one kv head; its four waves
-// take every fourth block of 32 keys, each with its own online softmax, and
-// merge in LDS.  All products are f32 on the matrix cores
-// (v_mfma_f32_16x16x4_f32).  Scores are formed transposed (keys x queries):
-// a lane then holds one query's scores, so the softmax factors are its own,
-// and the scores are already laid out as the operand of the value product.
+// take every fourth block of 32 keys, each with its own online softmax
+// (attn16.h), and merge in LDS.
 template <int HD> __global__ void __launch_bounds__(PWG) k_prompt_attn(PromptAttn a)
 {
-    constexpr int NQ = HD / 16, NV = HD / 64, DR = HD < 128 ? HD : 128;
-    constexpr int KT = 2, KB = 16 * KT;  // tiles and keys of a block
-    __shared__ __align__(16) float s_o[4][16][DR + 4];
-    __shared__ float s_m[4][16], s_l[4][16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
-    const int gqa = a.nh / a.nkv, kvh = blockIdx.y, nrow = a.T * gqa;
-    const int row = min((int)blockIdx.x * 16 + n, nrow - 1);
+    __shared__ __align__(16) Merge16<HD> s;
+    const int wave = threadIdx.x >> 6, n = threadIdx.x & 15;
+    const int gqa = a.nh / a.nkv, kvh = blockIdx.y, nrow = a.T * gqa, r0 = blockIdx.x * 16;
+    const int row = min(r0 + n, nrow - 1);
     const int tok = row / gqa, head = kvh * gqa + row % gqa, qpos = a.pos0 + tok;
-    const int last = a.pos0 + (min((int)blockIdx.x * 16 + 15, nrow - 1)) / gqa;  // largest key met
-    const float *qp = a.q + ((int64_t)tok * a.nh + head) * HD;
-    f4 q[NQ];
-#pragma unroll
-    for (int i = 0; i < NQ; i++) q[i] = *(const f4 *)(qp + 16 * i + 4 * g);
-    const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    f4 o[NV][4];
-#pragma unroll
-    for (int j = 0; j < NV; j++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) o[j][e] = zero;
-    float m = -INFINITY, l = 0.0f;
-    for (int k0 = wave * KB; k0 <= last; k0 += 4 * KB) {
-        // page_tokens is a multiple of KB: a key block lies in one page
+    const int last = a.pos0 + min(r0 + 15, nrow - 1) / gqa;  // largest key met
+    Attn16<HD> at;
+    at.init(a.q + ((int64_t)tok * a.nh + head) * HD);
+    for (int k0 = wave * A16_KB; k0 <= last; k0 += 4 * A16_KB) {
+        // page_tokens is a multiple of A16_KB: a key block lies in one page
         const int64_t pg = a.page_table[k0 / a.page_tokens];
         const int64_t base = ((pg * a.nkv + kvh) * a.page_tokens + k0 % a.page_tokens) * (int64_t)HD;
-        const int lim = last - k0;  // rows past the batch's last key are not read
-        float sc[KT][4], mn = m;
-#pragma unroll
-        for (int b = 0; b < KT; b++) {
-            const float *kp = a.kpool + base + (int64_t)min(16 * b + n, lim) * HD + 4 * g;
-            f4 s4[2][4];
-#pragma unroll
-            for (int i = 0; i < NQ; i++) {
-                const f4 kf = *(const f4 *)(kp + 16 * i);
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    s4[i & 1][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        kf[e], q[i][e], i < 2 ? zero : s4[i & 1][e], 0, 0, 0);
-            }
-            const f4 s = ((s4[0][0] + s4[0][1]) + (s4[0][2] + s4[0][3])) +
-                         ((s4[1][0] + s4[1][1]) + (s4[1][2] + s4[1][3]));
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                sc[b][i] = k0 + 16 * b + 4 * g + i <= qpos ? s[i] * a.scale : -INFINITY;
-                mn = fmaxf(mn, sc[b][i]);
-            }
-        }
-        {
-            const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(mn), __float_as_uint(mn), false, false);
-            mn = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
-            const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(mn), __float_as_uint(mn), false, false);
-            mn = fmaxf(__uint_as_float(y[0]), __uint_as_float(y[1]));
-        }
-        const float mz = mn == -INFINITY ? 0.0f : mn;  // no key of this query yet
-        const float corr = expf(m - mz);
-        m = mn;
-        float lb = 0.0f;
-#pragma unroll
-        for (int b = 0; b < KT; b++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) sc[b][i] = expf(sc[b][i] - mz);
-            lb += (sc[b][0] + sc[b][1]) + (sc[b][2] + sc[b][3]);
-        }
-        l = l * corr + lb;
-        // the block's value sum on its own, then added: the running sum is
-        // rounded once per block, not once per four keys
-        f4 ob[NV][4];
-#pragma unroll
-        for (int b = 0; b < KT; b++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float *vp = a.vpool + base + (int64_t)min(16 * b + 4 * g + i, lim) * HD + 4 * n;
-#pragma unroll
-                for (int j = 0; j < NV; j++) {
-                    const f4 v = *(const f4 *)(vp + 64 * j);
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        ob[j][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                            v[e], sc[b][i], b + i == 0 ? zero : ob[j][e], 0, 0, 0);
-                }
-            }
-#pragma unroll
-        for (int j = 0; j < NV; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) o[j][e] = o[j][e] * corr + ob[j][e];
+        at.block(a.kpool + base, a.vpool + base, HD, last - k0, qpos - k0 + 1, a.scale);
     }
-    // the query's sum over the four lane groups
-    {
-        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(l), __float_as_uint(l), false, false);
-        l = __uint_as_float(x[0]) + __uint_as_float(x[1]);
-        const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
-        l = __uint_as_float(y[0]) + __uint_as_float(y[1]);
-    }
-    if (g == 0) {
-        s_m[wave][n] = m;
-        s_l[wave][n] = l;
-    }
-#pragma unroll
-    for (int d0 = 0; d0 < HD; d0 += DR) {
-        __syncthreads();
-        // element (j, e), register i: value 64 j + 4 (4 g + i) + e of query n
-#pragma unroll
-        for (int j = d0 / 64; j < (d0 + DR) / 64; j++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const f4 v = {o[j][0][i], o[j][1][i], o[j][2][i], o[j][3][i]};
-                *(f4 *)&s_o[wave][n][64 * j - d0 + 4 * (4 * g + i)] = v;
-            }
-        __syncthreads();
-        for (int i = threadIdx.x; i < 16 * DR; i += PWG) {
-            const int r = i / DR, d = i % DR, qr = blockIdx.x * 16 + r;
-            if (qr >= nrow) break;
-            float M = s_m[0][r];
-            for (int w = 1; w < 4; w++) M = fmaxf(M, s_m[w][r]);
-            float L = 0.0f, O = 0.0f;
-            for (int w = 0; w < 4; w++) {
-                const float f = s_m[w][r] == -INFINITY ? 0.0f : expf(s_m[w][r] - M);
-                L += s_l[w][r] * f;
-                O += s_o[w][r][d] * f;
-            }
-            a.out[((int64_t)(qr / gqa) * a.nh + kvh * gqa + qr % gqa) * HD + d0 + d] = O / L;
-        }
-    }
+    attn16_merge<HD>(at, s, [&](int r, int d, float O, float L, float) {
+        const int qr = r0 + r;
+        if (qr < nrow) a.out[((int64_t)(qr / gqa) * a.nh + kvh * gqa + qr % gqa) * HD + d] = O / L;
+    });
 }
 
 static bool attn_ok(const PromptAttn &a)
 {
     return a.T >= 1 && a.nkv >= 1 && a.nh >= a.nkv && a.nh % a.nkv == 0 && a.pos0 >= 0 &&
-           (a.hd == 64 || a.hd == 128 || a.hd == 256) && a.page_tokens >= 32 && a.page_tokens % 32 == 0;
+           (a.hd == 64 || a.hd == 128 || a.hd == 256) && a.page_tokens >= A16_KB && a.page_tokens % A16_KB == 0;
 }
 
 hipError_t launch_prompt_rope(hipStream_t st, const PromptAttn &a)

@@ -28,6 +28,15 @@ enum RefKernel {
     RK_F_ATTN_PAGED = 76,
 };
 
+// Device scratch of the attention pipeline's chunk partials, used by the
+// launches of one call in stream order (p may be null: contexts are then not
+// split).
+struct RefScratch {
+    float *p;
+    uint64_t floats;
+};
+constexpr uint64_t REF_SCRATCH_FLOATS = 2u * 1024u * 1024u;
+
 // Launch reference kernel `kid` with resolved binding pointers and the bytes
 // each binding makes visible, the raw push-constant block, the reference
 // grid and spec constants (id, value pairs).  Returns hipErrorInvalidValue,
@@ -36,7 +45,7 @@ enum RefKernel {
 // binding are treated as SKIP by the kernels.
 hipError_t refk_launch(hipStream_t st, int kid, void *const *ptr, const uint64_t *size,
                        const void *push, uint32_t gx, uint32_t gy, uint32_t gz,
-                       const uint32_t *spec, int n_spec);
+                       const uint32_t *spec, int n_spec, const RefScratch *scratch);
 
 // Launch fused kernel `kid` (RK_F_*) of a batch on gpu g: the push block of
 // include/styx_hip.h, bindings resolved as for refk_launch.  Returns

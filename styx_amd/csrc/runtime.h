@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 
 #include "../../include/styx_hip.h"
@@ -36,6 +37,12 @@ struct styx_gpu {
     // outside the pools whatever the table holds.
     static constexpr int FUSED_PT_MAX = 65536;
     uint32_t *fused_pt = nullptr;
+    // Attention partials of batches on `stream` (refk.h RefScratch), made at
+    // the first one and kept; ref_mu is held over a dispatch's launches, so
+    // that batches of several threads do not come between a launch that
+    // writes the partials and the one that reads them.
+    float *ref_part = nullptr;
+    std::mutex ref_mu;
 };
 
 struct styx_buf {

@@ -1,0 +1,156 @@
+"""The reference pipelines' matvec, router matvec and attention kernels at
+the edges of their dispatch rules (styx_amd/csrc/kernels_ref.hip): row
+lengths around the lane groups, rows past the last pass, head groups that do
+not fill 16 rows, contexts around the split.  Against the oracle's f64
+results; matvecs within the f32 forward-error bound for any summation order
+(cols 2^-24 sum |w x|), attention within 2e-6 relative L2 (the bound the
+paged attention tests use)."""
+from __future__ import annotations
+
+import struct
+
+import numpy as np
+import pytest
+
+from helpers import clamp_f16_exponents, rel_l2
+from oracle import oracle as O
+from test_gpu_dispatch import BLK, F16_AT, NAME, f32buf, mmv_id_push, run, sum_bound
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    from styx_amd import Gpu
+    g = Gpu(0)
+    yield g
+    g.close()
+
+
+def weights(t, rows, cols, seed):
+    be, bb = BLK[t]
+    a = np.random.default_rng(seed).integers(0, 256, rows * (cols // be) * bb).astype(np.uint8)
+    clamp_f16_exponents(a, bb, F16_AT[t])
+    return a
+
+
+# lanes per row 1..64, one and two units per lane, rows longer than 128 units
+@pytest.mark.parametrize("t,rows,cols", [(8, 7, 32), (8, 130, 96), (8, 513, 2080), (8, 66, 6176),
+                                         (12, 9, 256), (12, 5001, 768), (12, 70, 4608),
+                                         (13, 33, 2304), (13, 259, 4096), (14, 65, 1280),
+                                         (14, 1030, 2048), (14, 35, 8192)])
+def test_matvec_rows(gpu, t, rows, cols):
+    be, _ = BLK[t]
+    a = weights(t, rows, cols, rows + cols)
+    x = np.random.default_rng(1).standard_normal(cols).astype(np.float32)
+    guard = 5
+    bd = f32buf(gpu, np.full(rows + guard, 9.0))
+    push = struct.pack("<13I", cols, cols // be, cols, rows, rows * cols, cols, rows, 0, 0, 1, 1, 1, 1)
+    run(gpu, f"mul_mat_vec_{NAME[t]}_f32_f32", [gpu.from_numpy(a), f32buf(gpu, x), bd, gpu.zeros(16),
+                                               gpu.zeros(16)], push, (rows, 1, 1), [(1, 1)])
+    got = bd.download(np.float32)
+    y = O.matvec_f64(t, a, rows, cols, x)
+    assert (np.abs(got[:rows] - y) <= sum_bound(t, a, rows, cols, x)).all()
+    assert (got[rows:] == 9.0).all()
+
+
+def test_matvec_grid_covers_part_of_the_rows(gpu):
+    """NUM_ROWS rows per workgroup of the reference grid, and no row past it."""
+    t, rows, cols = 12, 64, 512
+    a = weights(t, rows, cols, 3)
+    x = np.random.default_rng(2).standard_normal(cols).astype(np.float32)
+    bd = f32buf(gpu, np.full(rows, 9.0))
+    push = struct.pack("<13I", cols, 2, cols, rows, rows * cols, cols, rows, 0, 0, 1, 1, 1, 1)
+    run(gpu, "mul_mat_vec_q4_k_f32_f32", [gpu.from_numpy(a), f32buf(gpu, x), bd, gpu.zeros(16),
+                                          gpu.zeros(16)], push, (10, 1, 1), [(1, 4)])
+    got = bd.download(np.float32)
+    y = O.matvec_f64(t, a, rows, cols, x)
+    assert (np.abs(got - y)[:40] <= sum_bound(t, a, rows, cols, x)[:40]).all()
+    assert (got[40:] == 9.0).all()
+
+
+@pytest.mark.parametrize("t", [8, 12, 13, 14])
+def test_matvec_id_odd_stride(gpu, t):
+    """Activations a whole odd number of floats apart (4-byte aligned rows)."""
+    be, bb = BLK[t]
+    E, rows, cols, k, stride = 5, 37, 512, 3, 515
+    a = weights(t, E * rows, cols, 9 + t)
+    x = np.random.default_rng(4).standard_normal(k * stride).astype(np.float32)
+    bd = gpu.zeros(k * rows * 4)
+    ids = gpu.from_numpy(np.array([4, 0, 2], np.int32))
+    push = struct.pack("<12I", cols, cols // be, stride, rows, rows * cols, 0, k * rows, 0, k, k, 0, 1)
+    run(gpu, f"mul_mat_vec_id_{NAME[t]}_f32_f32", [gpu.from_numpy(a), f32buf(gpu, x), bd, gpu.zeros(16),
+                                                  gpu.zeros(16), ids], push, (rows, k, 1))
+    got = bd.download(np.float32).reshape(k, rows)
+    n = rows * (cols // be) * bb
+    for s, e in enumerate([4, 0, 2]):
+        xs = x[s * stride:s * stride + cols]
+        w = a[e * n:(e + 1) * n]
+        assert (np.abs(got[s] - O.matvec_f64(t, w, rows, cols, xs)) <= sum_bound(t, w, rows, cols, xs)).all()
+
+
+@pytest.mark.parametrize("E,H,stride", [(1, 3, 3), (17, 259, 261), (16, 2048, 2048), (33, 2563, 2567),
+                                        (8, 4352, 4352)])
+def test_matvec_strided_shapes(gpu, E, H, stride):
+    rng = np.random.default_rng(H)
+    W = rng.standard_normal(E * stride).astype(np.float32)
+    x = rng.standard_normal(H).astype(np.float32)
+    bd = gpu.zeros(E * 4)
+    run(gpu, "matvec_strided_f32", [f32buf(gpu, W), f32buf(gpu, x), bd], struct.pack("<2I", H, stride),
+        (E, 1, 1))
+    Wd = W.reshape(E, stride)[:, :H].astype(np.float64)
+    bound = H * 2.0 ** -24 * (np.abs(Wd) @ np.abs(x.astype(np.float64)))
+    assert (np.abs(bd.download(np.float32, E) - Wd @ x.astype(np.float64)) <= bound).all()
+
+
+# contexts around a key block (32), a workgroup's pass (128), the split (256)
+# and past one chunk per workgroup; 1..20 heads per kv head, and a head count
+# that leaves the last kv head's group short; rows of an odd stride
+@pytest.mark.parametrize("n_t,hd,nh,gqa,pad", [
+    (1, 64, 4, 1, 0), (31, 128, 8, 8, 0), (33, 256, 6, 3, 0), (129, 64, 20, 20, 0), (256, 128, 32, 8, 0),
+    (257, 128, 32, 8, 0), (300, 256, 16, 16, 0), (1000, 64, 7, 4, 0), (1023, 128, 10, 5, 1),
+    (9000, 64, 2, 1, 0), (700, 96, 8, 4, 0)])
+def test_attn_decode_shapes(gpu, n_t, hd, nh, gqa, pad):
+    rng = np.random.default_rng(n_t + hd)
+    nkv = -(-nh // gqa)
+    kvd = nkv * hd + pad
+    q = rng.standard_normal(nh * hd).astype(np.float32)
+    K = rng.standard_normal(n_t * kvd).astype(np.float32)
+    V = rng.standard_normal(n_t * kvd).astype(np.float32)
+    scale = np.float32(1 / np.sqrt(hd))
+    bo = f32buf(gpu, np.full(nh * hd + 8, 3.0))
+    run(gpu, "attn_decode_f32", [f32buf(gpu, q), f32buf(gpu, K), f32buf(gpu, V), bo],
+        struct.pack("<4If", n_t, hd, kvd, gqa, scale), (nh, 1, 1))
+    got = bo.download(np.float32)
+    ref = O.attn_decode_f64(q, K, V, n_t, hd, kvd, gqa, nh, float(scale))
+    assert rel_l2(got[:nh * hd], ref) < 2e-6
+    assert (got[nh * hd:] == 3.0).all()
+
+
+def test_attn_in_async_and_plain_batches(gpu):
+    """Split contexts on two streams at once: each batch has its own partials."""
+    from styx_amd.runtime import Batch, Kernel, Timeline
+    rng = np.random.default_rng(8)
+    n_t, hd, nh, nkv = 2000, 128, 8, 2
+    kvd, scale = nkv * hd, np.float32(1 / np.sqrt(hd))
+    push = struct.pack("<4If", n_t, hd, kvd, nh // nkv, scale)
+    k = Kernel(gpu, "attn_decode_f32", [])
+    t, ab, mb = Timeline(gpu), Batch(gpu, is_async=True), Batch(gpu)
+    sets = []
+    for _ in range(2):
+        q, K, V = (rng.standard_normal(n).astype(np.float32) for n in (nh * hd, n_t * kvd, n_t * kvd))
+        ref = O.attn_decode_f64(q, K, V, n_t, hd, kvd, nh // nkv, nh, float(scale))
+        sets.append(([f32buf(gpu, q), f32buf(gpu, K), f32buf(gpu, V), gpu.zeros(nh * hd * 4)], ref))
+    for rnd in range(4):
+        ab.begin()
+        mb.begin()
+        for _ in range(4):
+            ab.dispatch(k, sets[0][0], push, (nh, 1, 1))
+            mb.dispatch(k, sets[1][0], push, (nh, 1, 1))
+        ab.submit_async(t, rnd + 1)
+        mb.submit()
+        ab.wait_idle()
+        for binds, ref in sets:
+            assert rel_l2(binds[3].download(np.float32), ref) < 2e-6
+    for o in (ab, mb, k, t):
+        o.free()
