@@ -357,14 +357,12 @@ __device__ __forceinline__ void u4v_to(const styx_u4 v, uint32_t *o)
     o[0] = v.x, o[1] = v.y, o[2] = v.z, o[3] = v.w;
 }
 
-template <int T, bool D8, int NG, int TT>
-__device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], const uint8_t *xl, int tm,
-                                          const uint8_t *sl, f4 (&acc)[NG][TT])
+// acc += the products of a step: xop(t, piece, s) gives the activation
+// operand of token tile t, sop(t) its run sums' (q4_K, q5_K).
+template <int T, bool D8, int NG, int TT, typename XOp, typename SOp>
+__device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp sop, f4 (&acc)[NG][TT])
 {
-    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-    auto xop = [&](int t, int piece, int s) {
-        return *(const h8 *)(xl + (piece * tm + 16 * t + n) * XROW + 16 * x_run<T>(g, s));
-    };
+    const int lane = threadIdx.x & 63, g = lane >> 4;
     auto mm = [](h8 a, h8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); };
     const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (T == T_Q8_0) {
@@ -520,7 +518,7 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], const uint8_
                 const float d = f16f(w[r].hd.x), dm = -64.0f * f16f(w[r].hd.x >> 16);
 #pragma unroll
                 for (int t = 0; t < TT; t++) {
-                    const f4 mn = mm(*(const h8 *)(sl + (16 * t + n) * 64 + 16 * g), mv, zero);
+                    const f4 mn = mm(sop(t), mv, zero);
                     acc[r][t] += d * (big[r][t] + small[r][t]) + dm * mn;
                 }
             }
@@ -636,7 +634,12 @@ __global__ void __launch_bounds__(PWG, 2) k_prompt_gemm(PromptGemm a)
             wload(c + 1);
             xload(c + 1);
         }
-        gemm_step<T, D8, NG, TT>(wc, s_x, TM, s_sum, acc);
+        gemm_step<T, D8, NG, TT>(
+            wc,
+            [&](int t, int p, int s) {
+                return *(const h8 *)(s_x + (p * TM + 16 * t + n) * XROW + 16 * x_run<T>(g, s));
+            },
+            [&](int t) { return *(const h8 *)(s_sum + (16 * t + n) * 64 + 16 * g); }, acc);
     }
 #pragma unroll
     for (int t = 0; t < TT; t++)
@@ -654,6 +657,89 @@ __global__ void __launch_bounds__(PWG, 2) k_prompt_gemm(PromptGemm a)
                 *y = a.add ? *y + v : v;
             }
         }
+}
+
+// The same for a dense matrix and at most 32 positions, 16 rows per
+// workgroup: each wave takes every fourth step of the columns with its
+// activations straight from the L2, and the waves' sums meet in LDS.  A
+// workgroup of the kernel above walks all steps in turn, each a memory round
+// trip of about 3 us while few workgroups share a CU: q8_0 q/k/v (5120 x
+// 2048) 26 us at 9 and 19 tokens, here 15 and 23; o-proj (2048 x 4096) 48,
+// here 16 and 24; k/v (1024 x 2048) 25, here 8 and 12.  From 33 tokens on the
+// activations' L2 traffic (every workgroup reads them all) outweighs it.
+template <int T, bool D8, int TT> __global__ void __launch_bounds__(PWG, 2) k_prompt_gemm_few(PromptGemm a)
+{
+    __shared__ f4 s_acc[4][TT][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+    int rt = blockIdx.x, seg = 0;
+    while (seg + 1 < a.nseg && rt >= a.rt0[seg + 1]) seg++;
+    rt -= a.rt0[seg];
+    const int rows = a.rows[seg], nb = a.x.n / blk_elems(T), nc = a.x.np / KC;
+    const Split sl = split_of(T);
+    const int64_t nblk = (int64_t)rows * nb;
+    const Buf m(a.w[seg], nblk * blk_bytes(T));
+    const Reg ro{(uint32_t)region_off(sl, 1, nblk), (uint32_t)region_off(sl, 2, nblk),
+                 (uint32_t)region_off(sl, 3, nblk)};
+    const int64_t plane = a.x.rows * (int64_t)a.x.np * 2;
+    const Buf xb[3] = {{a.x.p, plane}, {(const uint8_t *)a.x.p + plane, plane}, {(const uint8_t *)a.x.p + 2 * plane, plane}};
+    const Buf sb(a.x.sums, a.x.rows * nc * 64);
+    uint32_t xo[TT], so[TT];
+#pragma unroll
+    for (int t = 0; t < TT; t++) {
+        const uint32_t row = min(16 * t + n, a.T - 1);
+        xo[t] = row * a.x.np * 2;
+        so[t] = row * nc * 64 + 16 * g;
+    }
+    const uint32_t row = min(rt * 16 + n, rows - 1);
+    f4 acc[1][TT];
+#pragma unroll
+    for (int t = 0; t < TT; t++) acc[0][t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c = wave; c < nc; c += 4) {
+        // every load of the step before any product: one round trip a step
+        PW<T, D8> w[1];
+        w[0].load(m, ro, row, nb, c, g);
+        styx_u4 x[TT][3][8], xs[TT];
+#pragma unroll
+        for (int t = 0; t < TT; t++) {
+#pragma unroll
+            for (int s = 0; s < 8; s++)
+#pragma unroll
+                for (int p = 0; p < 3; p++) x[t][p][s] = xb[p].b128(xo[t] + 16 * x_run<T>(g, s), c * KC * 2);
+            if (T == T_Q4_K || T == T_Q5_K) xs[t] = sb.b128(so[t], c * 64);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        gemm_step<T, D8, 1, TT>(
+            w, [&](int t, int p, int s) { return __builtin_bit_cast(h8, x[t][p][s]); },
+            [&](int t) { return __builtin_bit_cast(h8, xs[t]); }, acc);
+    }
+#pragma unroll
+    for (int t = 0; t < TT; t++) s_acc[wave][t][lane] = acc[0][t];
+    __syncthreads();
+    if (wave >= TT) return;
+    const int t = wave;
+    const f4 v = (s_acc[0][t][lane] + s_acc[1][t][lane]) + (s_acc[2][t][lane] + s_acc[3][t][lane]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int p = 16 * t + 4 * g + i;
+        if (p >= a.T || rt * 16 + n >= rows) continue;
+        float *y = a.y[seg] + (int64_t)p * rows + rt * 16 + n;
+        const float r = v[i] * a.x.scale[p];
+        *y = a.add ? *y + r : r;
+    }
+}
+
+template <int T, bool D8> static hipError_t gemm_few(hipStream_t st, PromptGemm &a)
+{
+    a.nrt = 0;
+    for (int s = 0; s < a.nseg; s++) {
+        a.rt0[s] = a.nrt;
+        a.nrt += (a.rows[s] + 15) / 16;
+    }
+    if (a.T <= 16)
+        hipLaunchKernelGGL((k_prompt_gemm_few<T, D8, 1>), dim3(a.nrt), dim3(PWG), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_prompt_gemm_few<T, D8, 2>), dim3(a.nrt), dim3(PWG), 0, st, a);
+    return hipGetLastError();
 }
 
 template <int T, bool D8, int TT, int NG> static hipError_t gemm_go(hipStream_t st, PromptGemm &a)
@@ -677,6 +763,7 @@ template <int T, bool D8 = true> static hipError_t gemm_t(hipStream_t st, Prompt
     // (each activation operand read from LDS serves both) unless that would
     // leave CUs without a workgroup
     const int64_t rows = (int64_t)a.rows[0] + (a.nseg > 1 ? a.rows[1] : 0) + (a.nseg > 2 ? a.rows[2] : 0);
+    if (!a.tiles && a.T <= 32) return gemm_few<T, D8>(st, a);
     const int tm = a.tile_tokens;
     const int64_t wg2 = (rows + 127) / 128 * (a.tiles ? a.max_tiles : (a.T + tm - 1) / tm);
     if (tm == 16) return wg2 < 256 ? gemm_go<T, D8, 1, 1>(st, a) : gemm_go<T, D8, 1, 2>(st, a);
