@@ -6,84 +6,6 @@
 
 namespace styx {
 
-// --------------------------------------------------------- top-k softmax --
-// topk_softmax_f32.comp:29-67 on one wave64: softmax max/sum, then k rounds
-// of argmax over untaken entries (ties -> lowest index), weights
-// exp(best-mx)/sum, renormalised by their sum if renorm.  Id rows:
-// [0,k) original, [16,..) hot, [32,..) arena, [48,..) host.
-// remap == nullptr means every expert is resident at its own index.
-__device__ __noinline__ void topk_wave(const float *logits, int n, int k, int renorm,
-                                 const uint32_t *remap, const uint32_t *pmap, int arena_mode,
-                                 int layer, float *wts, int32_t *ids)
-{
-    const int lane = threadIdx.x & 63;
-    float v[MAX_EXPERTS / 64];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < MAX_EXPERTS / 64; j++) {
-        const int i = lane + 64 * j;
-        v[j] = i < n ? logits[i] : -INFINITY;
-        mx = fmaxf(mx, v[j]);
-    }
-    mx = wave_max(mx);
-    float sum = 0.0f;
-#pragma unroll
-    for (int j = 0; j < MAX_EXPERTS / 64; j++)
-        if (lane + 64 * j < n) sum += expf(v[j] - mx);
-    sum = wave_sum(sum);
-
-    uint32_t taken = 0;
-    float my_w = 0.0f, wsum = 0.0f;
-    int my_id = -1;
-    for (int s = 0; s < k; s++) {
-        float best = -INFINITY;
-        int bi = 0x7FFFFFFF;
-#pragma unroll
-        for (int j = 0; j < MAX_EXPERTS / 64; j++) {
-            const int i = lane + 64 * j;
-            if (i < n && !((taken >> j) & 1u) && v[j] > best) {
-                best = v[j];
-                bi = i;
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ob = __shfl_xor(best, o);
-            const int oi = __shfl_xor(bi, o);
-            if (ob > best || (ob == best && oi < bi)) {
-                best = ob;
-                bi = oi;
-            }
-        }
-        if (bi != 0x7FFFFFFF && lane == (bi & 63)) taken |= 1u << (bi >> 6);
-        const float w = expf(best - mx) / sum;
-        wsum += w;
-        if (lane == s) {
-            my_w = w;
-            my_id = bi;
-        }
-    }
-    if (lane < k) {
-        wts[lane] = renorm ? my_w / wsum : my_w;
-        const uint32_t e = (uint32_t)my_id;
-        ids[lane] = my_id;
-        const uint32_t h = remap ? remap[e] : e;
-        if (h != SKIP) {
-            ids[16 + lane] = (int32_t)h;
-            ids[32 + lane] = (int32_t)SKIP;
-            ids[48 + lane] = (int32_t)SKIP;
-        } else {
-            uint32_t a = SKIP;
-            if (arena_mode)
-                a = (uint32_t)(layer * k + lane);
-            else if (pmap)
-                a = pmap[e];
-            ids[16 + lane] = (int32_t)SKIP;
-            ids[32 + lane] = (int32_t)a;
-            ids[48 + lane] = a != SKIP ? (int32_t)SKIP : my_id;
-        }
-    }
-}
-
 // Hot / arena / host ids of expert e routed to `slot` (topk_softmax_f32.comp
 // id rows 16/32/48): the hot slot from remap (every expert resident at its
 // own index when remap is null), else an arena slot (arena_mode: layer*k +
@@ -155,6 +77,101 @@ __device__ __forceinline__ uint64_t wave_max_key(uint64_t v)
     else
         ml = wave_max_u32(hi == mh ? (uint32_t)v : 0u);
     return join64(mh, ml);
+}
+
+// --------------------------------------------------------- top-k softmax --
+// topk_softmax_f32.comp:29-67 on one wave64: softmax max/sum, then k rounds
+// of argmax over untaken entries (ties -> lowest index), weights
+// exp(best-mx)/sum, renormalised by their sum if renorm.  Id rows:
+// [0,k) original, [16,..) hot, [32,..) arena, [48,..) host.
+// remap == nullptr means every expert is resident at its own index.
+//
+// One wave, so a round's time is its chain of dependent operations: the
+// argmax is the wave's largest rank key (wave_max_key, lane permutes in the
+// VALU), the lane that holds it drops it, and only the NV = n / 64 keys a
+// lane holds are looked at; weights are formed once, after the rounds.  With
+// two LDS permutes per step of each round's reduction, 8 slots per lane
+// whatever n, the launch for 128 experts (k = 8) took 8.8 us, so 4.4.  Entries that no
+// comparison with -inf finds larger (-inf, NaN) hold key 0 and are never
+// picked; with none left the id is 0x7FFFFFFF.
+template <int NV>
+__device__ __forceinline__ void topk_wave_n(const float *logits, int n, int k, int renorm,
+                                            const uint32_t *remap, const uint32_t *pmap,
+                                            int arena_mode, int layer, float *wts, int32_t *ids)
+{
+    const int lane = threadIdx.x & 63;
+    float v[NV];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = lane + 64 * j;
+        v[j] = i < n ? logits[i] : -INFINITY;
+        mx = fmaxf(mx, v[j]);
+    }
+    mx = wave_max(mx);
+    float sum = 0.0f;
+    uint64_t key[NV], best = 0;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        if (lane + 64 * j < n) sum += expf(v[j] - mx);
+        key[j] = v[j] > -INFINITY ? rank_key(v[j], lane + 64 * j) : 0;
+        best = max(best, key[j]);
+    }
+    sum = wave_sum(sum);
+
+    uint64_t mine = 0;
+    for (int s = 0; s < k; s++) {
+        const uint64_t m = wave_max_key(best);
+        if (lane == s) mine = m;
+        best = 0;
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            if (key[j] == m) key[j] = 0;
+            best = max(best, key[j]);
+        }
+    }
+    // the lane's pick and its weight
+    const uint32_t hi = (uint32_t)(mine >> 32);
+    const float pick = mine ? __uint_as_float(hi & 0x80000000u ? hi ^ 0x80000000u : ~hi) : -INFINITY;
+    const int my_id = mine ? (int)(0xFFFFFFFFu - (uint32_t)mine) : 0x7FFFFFFF;
+    const float my_w = expf(pick - mx) / sum;
+    float wsum = 0.0f;
+    for (int s = 0; s < k; s++)
+        wsum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_w), s));
+    if (lane < k) {
+        wts[lane] = renorm ? my_w / wsum : my_w;
+        const uint32_t e = (uint32_t)my_id;
+        ids[lane] = my_id;
+        const uint32_t h = !remap ? e : mine ? remap[e] : SKIP;
+        if (h != SKIP) {
+            ids[16 + lane] = (int32_t)h;
+            ids[32 + lane] = (int32_t)SKIP;
+            ids[48 + lane] = (int32_t)SKIP;
+        } else {
+            uint32_t a = SKIP;
+            if (arena_mode)
+                a = (uint32_t)(layer * k + lane);
+            else if (pmap && mine)
+                a = pmap[e];
+            ids[16 + lane] = (int32_t)SKIP;
+            ids[32 + lane] = (int32_t)a;
+            ids[48 + lane] = a != SKIP ? (int32_t)SKIP : my_id;
+        }
+    }
+}
+
+__device__ __noinline__ void topk_wave(const float *logits, int n, int k, int renorm,
+                                       const uint32_t *remap, const uint32_t *pmap, int arena_mode,
+                                       int layer, float *wts, int32_t *ids)
+{
+    if (n <= 64)
+        topk_wave_n<1>(logits, n, k, renorm, remap, pmap, arena_mode, layer, wts, ids);
+    else if (n <= 128)
+        topk_wave_n<2>(logits, n, k, renorm, remap, pmap, arena_mode, layer, wts, ids);
+    else if (n <= 256)
+        topk_wave_n<4>(logits, n, k, renorm, remap, pmap, arena_mode, layer, wts, ids);
+    else
+        topk_wave_n<MAX_EXPERTS / 64>(logits, n, k, renorm, remap, pmap, arena_mode, layer, wts, ids);
 }
 
 // Stage 1 of the two-stage ranking for one wave: the Q keys of its quarter
