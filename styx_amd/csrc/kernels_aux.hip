@@ -10,10 +10,96 @@
 namespace styx {
 
 // ------------------------------------------------- GGUF <-> split layout --
-// One thread per block; each region's bytes are moved with byte loops (a
-// load-time operation).
-__global__ void k_to_split(int t, const uint8_t *src, uint8_t *dst, int64_t nblocks, int64_t nmat,
-                           int dir)
+// 16-byte word o / 16 of region r of a tile of blocks: its 16 bytes are those
+// at `byte` of block `blk` in GGUF order (ilv_off inverted).  Regions of 2
+// bytes per block (f16 factors) hold 8 blocks' factors per word instead.
+template <int T> __device__ __forceinline__ void split_word(int r, int o, int &blk, int &byte)
+{
+    const int rem = o & 255, k = (rem >> 4) & 3;
+    if (r == 0 && (T == T_Q4_K || T == T_Q5_K)) {
+        blk = 2 * (o >> 8) + ((rem >> 6) & 1);
+        byte = 32 * k + 16 * (rem >> 7);
+    } else if (r == 0 && T == T_Q6_K) {
+        blk = 2 * (o >> 8) + ((rem >> 6) & 1);
+        byte = 64 * (k >> 1) + 32 * (rem >> 7) + 16 * (k & 1);
+    } else if ((r == 0 && T == T_Q8_0) || (r == 1 && T == T_Q5_K)) {
+        blk = 8 * (o >> 8) + ((rem >> 4) & 7);
+        byte = 16 * (rem >> 7);
+    } else {
+        const int sz = split_of(T).sz[r];  // 16 or 64
+        blk = o / sz;
+        byte = o % sz;
+    }
+}
+
+// A tile of SPLIT_TILE blocks of one matrix through LDS: the GGUF side is
+// one contiguous run, the split side one run per region, both in 16-byte
+// words.  Bound: a copy of the tensor.  Matrices of whole groups of 8 blocks
+// at 16-byte aligned addresses (every model tensor; the others take
+// k_split_any).  128 q4_K slabs of 768 x 2048 (226 MB moved): 900 us by
+// bytes, one thread per block; 46 us so (4.9 TB/s, the rate of a copy).
+constexpr int SPLIT_TILE = 128;
+template <int T, int DIR>
+__global__ void __launch_bounds__(256) k_split_tile(const uint8_t *src, uint8_t *dst, int64_t nblocks,
+                                                    int64_t tiles, int64_t ntile)
+{
+    constexpr int bb = T == T_Q8_0 ? 34 : T == T_Q4_K ? 144 : T == T_Q5_K ? 176 : 210;
+    struct __attribute__((packed, aligned(2))) U16 { uint32_t w[4]; };
+    __shared__ __align__(16) uint8_t s_t[SPLIT_TILE * bb];
+    const Split s = split_of(T);
+    for (int64_t it = blockIdx.x; it < ntile; it += gridDim.x) {
+        const int64_t m = it / tiles, b0 = (it - m * tiles) * SPLIT_TILE;
+        const int nb = (int)min((int64_t)SPLIT_TILE, nblocks - b0);
+        const int64_t mbase = m * nblocks * bb;
+        const styx_u4 *g = (const styx_u4 *)((DIR == 0 ? src : dst) + mbase + b0 * bb);
+        if (DIR == 0) {
+            for (int i = threadIdx.x; i < nb * bb / 16; i += 256) ((styx_u4 *)s_t)[i] = g[i];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            if (r >= s.nreg) break;
+            const int64_t base = mbase + region_off(s, r, nblocks) + b0 * s.sz[r];
+            for (int i = threadIdx.x; i < nb * s.sz[r] / 16; i += 256) {
+                if (s.sz[r] == 2) {
+                    uint16_t h[8];
+                    if (DIR == 0) {
+#pragma unroll
+                        for (int j = 0; j < 8; j++) h[j] = *(const uint16_t *)(s_t + (8 * i + j) * bb + s.src[r]);
+                        styx_u4 v;
+#pragma unroll
+                        for (int j = 0; j < 4; j++) v[j] = h[2 * j] | (uint32_t)h[2 * j + 1] << 16;
+                        *(styx_u4 *)(dst + base + 16 * i) = v;
+                    } else {
+                        const styx_u4 v = *(const styx_u4 *)(src + base + 16 * i);
+#pragma unroll
+                        for (int j = 0; j < 8; j++)
+                            *(uint16_t *)(s_t + (8 * i + j) * bb + s.src[r]) = (uint16_t)(v[j / 2] >> (16 * (j & 1)));
+                    }
+                    continue;
+                }
+                int blk, byte;
+                split_word<T>(r, 16 * i, blk, byte);
+                U16 *t = (U16 *)(s_t + blk * bb + s.src[r] + byte);
+                if (DIR == 0) {
+                    *(styx_u4 *)(dst + base + 16 * i) = styx_u4{t->w[0], t->w[1], t->w[2], t->w[3]};
+                } else {
+                    const styx_u4 v = *(const styx_u4 *)(src + base + 16 * i);
+                    *t = U16{{v.x, v.y, v.z, v.w}};
+                }
+            }
+        }
+        __syncthreads();
+        if (DIR == 1) {
+            for (int i = threadIdx.x; i < nb * bb / 16; i += 256) ((styx_u4 *)g)[i] = ((styx_u4 *)s_t)[i];
+            __syncthreads();
+        }
+    }
+}
+
+// Any block count and alignment: one thread per block, byte by byte.
+__global__ void k_split_any(int t, const uint8_t *src, uint8_t *dst, int64_t nblocks, int64_t nmat,
+                            int dir)
 {
     const Split s = split_of(t);
     const int bb = blk_bytes(t);
@@ -21,8 +107,6 @@ __global__ void k_to_split(int t, const uint8_t *src, uint8_t *dst, int64_t nblo
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
          i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t m = i / nblocks, b = i - m * nblocks;
-        const uint8_t *gs = (dir ? dst : src);
-        (void)gs;
         const int64_t mbase = m * nblocks * bb;
         for (int r = 0; r < s.nreg; r++) {
             const int64_t so = mbase + b * bb + s.src[r];
@@ -35,14 +119,35 @@ __global__ void k_to_split(int t, const uint8_t *src, uint8_t *dst, int64_t nblo
     }
 }
 
+template <int T>
+static void split_tiles(hipStream_t st, const uint8_t *src, uint8_t *dst, int64_t nblocks, int64_t nmat,
+                        int dir)
+{
+    const int64_t tiles = (nblocks + SPLIT_TILE - 1) / SPLIT_TILE, n = tiles * nmat;
+    const dim3 grid((unsigned)std::min<int64_t>(n, 1 << 20));
+    if (dir == 0)
+        hipLaunchKernelGGL((k_split_tile<T, 0>), grid, dim3(256), 0, st, src, dst, nblocks, tiles, n);
+    else
+        hipLaunchKernelGGL((k_split_tile<T, 1>), grid, dim3(256), 0, st, src, dst, nblocks, tiles, n);
+}
+
 static hipError_t split_launch(hipStream_t st, int t, const uint8_t *src, uint8_t *dst,
                                int64_t nblocks, int64_t nmat, int dir)
 {
     if (blk_bytes(t) == 0 || nblocks < 1 || nmat < 1 || nblocks % ilv_group(t))
         return hipErrorInvalidValue;
+    if (nblocks % 8 == 0 && (((uintptr_t)src | (uintptr_t)dst) & 15) == 0 && is_quant(t)) {
+        switch (t) {
+        case T_Q8_0: split_tiles<T_Q8_0>(st, src, dst, nblocks, nmat, dir); break;
+        case T_Q4_K: split_tiles<T_Q4_K>(st, src, dst, nblocks, nmat, dir); break;
+        case T_Q5_K: split_tiles<T_Q5_K>(st, src, dst, nblocks, nmat, dir); break;
+        default: split_tiles<T_Q6_K>(st, src, dst, nblocks, nmat, dir); break;
+        }
+        return hipGetLastError();
+    }
     const int64_t total = nblocks * nmat;
     const int64_t nwg = std::min<int64_t>((total + 255) / 256, 65536);
-    hipLaunchKernelGGL(k_to_split, dim3((unsigned)std::max<int64_t>(nwg, 1)), dim3(256), 0, st, t,
+    hipLaunchKernelGGL(k_split_any, dim3((unsigned)std::max<int64_t>(nwg, 1)), dim3(256), 0, st, t,
                        src, dst, nblocks, nmat, dir);
     return hipGetLastError();
 }
