@@ -280,9 +280,8 @@ int styx_op_matvec(styx_gpu *g, int type, const void *w, int nrows, int ncols, c
         return fail(STYX_E_INVALID, "styx_op_matvec: bad shape");
     if (!w || !x || !y) return fail(STYX_E_INVALID, "styx_op_matvec: NULL pointer");
     const Xq q = xq_at(g->xq_scratch, ncols);
-    OP_RUN(launch_xq(g->stream, x, nullptr, norm_w, eps, ncols, q, nullptr), "styx_op_matvec");
-    DenseSeg s{(const uint8_t *)w, y, nrows};
-    OP_RUN(launch_dense(g->stream, type, ncols, &s, 1, q, add), "styx_op_matvec");
+    OP_RUN(launch_dense_f32(g->stream, type, (const uint8_t *)w, nrows, ncols, x, norm_w, eps, y, add, q),
+           "styx_op_matvec");
     return STYX_OK;
 }
 
@@ -349,9 +348,8 @@ int styx_op_moe_gate_up(styx_gpu *g, int tg, int tu, const styx_expert_src *gate
         return fail(STYX_E_INVALID, "styx_op_moe_gate_up: bad argument");
     if (H < 32 || H % 32 || H > XQ_MAX) return fail(STYX_E_INVALID, "styx_op_moe_gate_up: bad H");
     const Xq q = xq_at(g->xq_scratch, H);
-    OP_RUN(launch_xq(g->stream, xn, nullptr, nullptr, 0.0f, H, q, nullptr), "styx_op_moe_gate_up");
     OP_RUN(launch_moe_gate_up(g->stream, tg, tu, to_src(gate), to_src(up), ids, nullptr, q, gu, H,
-                              F, k),
+                              F, k, nullptr, nullptr, SLOTS_ALL, xn),
            "styx_op_moe_gate_up");
     return STYX_OK;
 }

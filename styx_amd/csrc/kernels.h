@@ -44,6 +44,13 @@ hipError_t launch_dense(hipStream_t st, int t, int ncols, const DenseSeg *segs, 
                         const Xq &xq, int add, const NormScale *ns = nullptr,
                         unsigned long long *amax = nullptr);
 
+// y = W . xn (add: y += W . xn), xn = x or rmsnorm(x) * norm_w, every
+// workgroup building the limbs of xn itself; scratch: limbs of ncols values,
+// used when y overlaps the inputs.
+hipError_t launch_dense_f32(hipStream_t st, int t, const uint8_t *w, int nrows, int ncols,
+                            const float *x, const float *norm_w, float eps, float *y, int add,
+                            const Xq &scratch);
+
 // Router for one layer (fused ffn_norm): writes logits[E] and, from its first
 // workgroup, xn (f32) and its limbs xq (if xq.A).  launch_router_topk also
 // runs the top-k into weights[k] and the 64-int id row.
@@ -79,6 +86,8 @@ hipError_t launch_topk_softmax(hipStream_t st, const float *logits, int n, int k
 // given by its limbs; routing from `route` (ranked in-kernel) or, if null,
 // the id row `ids`.  With sh_gate/sh_up (split-layout matrices of the same
 // types and width F) the shared expert is slot k: gu is [2][k+1][F].
+// With x (ids given, no route) the vector is x [H] in f32 and every
+// workgroup builds its limbs; xq is then scratch for them.
 // Slot filter of the expert kernels: every routed slot, only the slots whose
 // expert is hot (in HBM; the shared expert counts as hot), or only the
 // others (arena / host).  A filtered-out slot's outputs are left untouched,
@@ -88,7 +97,8 @@ enum SlotFilter { SLOTS_ALL = 0, SLOTS_HOT = 1, SLOTS_COLD = 2 };
 hipError_t launch_moe_gate_up(hipStream_t st, int tg, int tu, const ExpSrc &g, const ExpSrc &u,
                               const int32_t *ids, const Route *route, const Xq &xq, float *gu,
                               int H, int F, int k, const uint8_t *sh_gate = nullptr,
-                              const uint8_t *sh_up = nullptr, int filter = SLOTS_ALL);
+                              const uint8_t *sh_up = nullptr, int filter = SLOTS_ALL,
+                              const float *x = nullptr);
 
 // h[s] = swiglu(Wg[e_s] xn, Wu[e_s] xn) for the k slots, e_s = ids[s] (one
 // id per slot; an id at or past n_slabs, SKIP among them, leaves h[s]

@@ -122,7 +122,58 @@ hipError_t launch_xq(hipStream_t st, const float *x, const float *u, const float
     return hipGetLastError();
 }
 
+// An f32 vector whose limbs a matvec's workgroups build for themselves (in
+// LDS, of x or of rmsnorm(x) * nw), instead of reading those of a k_xq launch
+// in front: the op entry points' form.  Vectors of up to 8 values per thread
+// are loaded at entry, before the first weights, and turned into limbs while
+// these are in flight; longer ones are read by xq_build.
+struct XRaw {
+    const float *x, *nw;
+    float eps;
+};
+struct XBuild {
+    float4 x[2], w[2];
+    __device__ __forceinline__ void load(const XRaw &r, int n)
+    {
+        if (n > 8 * WG) return;
+        const int i = min(8 * (int)threadIdx.x, n - 8);
+        const float4 *p = (const float4 *)(r.x + i), *q = (const float4 *)((r.nw ? r.nw : r.x) + i);
+        x[0] = p[0], x[1] = p[1], w[0] = q[0], w[1] = q[1];
+    }
+    __device__ __forceinline__ void limbs(const XRaw &r, int n, const Xq &q, float *red) const
+    {
+        if (n > 8 * WG) {
+            xq_build<WG>(r.x, r.nw, r.eps, r.nw != nullptr, n, q, red, nullptr);
+        } else {
+            const int g = threadIdx.x;
+            const bool act = 8 * g < n;
+            float v[8] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w};
+            const float u[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
+            float ss = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                if (!act) v[i] = 0.0f;
+                ss += v[i] * v[i];
+            }
+            if (r.nw) {
+                const float scale = 1.0f / sqrtf(block_sum<WG>(ss, red) / (float)n + r.eps);
+#pragma unroll
+                for (int i = 0; i < 8; i++) v[i] = (v[i] * scale) * u[i];
+            }
+            xq_group(v, act, g, q);
+        }
+        __syncthreads();
+    }
+};
+// Whether [a, a + na) and [b, b + nb) share a float (the building workgroups
+// read x while others write y).
+static bool overlap(const float *a, int64_t na, const float *b, int64_t nb)
+{
+    return a && b && a < b + nb && b < a + na;
+}
+
 // ------------------------------------------------------------------ dense --
+enum XMode { X_LIMBS = 0, X_STAGE = 1, X_BUILD = 2 };
 struct DenseK {
     const uint8_t *w[3];
     float *y[3];
@@ -131,6 +182,7 @@ struct DenseK {
     Xq xq;
     NormScale ns;  // ns.ss == null: no RMSNorm scale
     unsigned long long *amax;  // optional: running argmax word (argmax_key)
+    XRaw raw;  // X_BUILD: the vector (xq unused)
 };
 
 // Rows per lane group and batch of the dense walk: two batches are in
@@ -140,15 +192,17 @@ template <int UPL> constexpr int dense_nr() { return UPL <= 2 ? 2 : 1; }
 // GC: the lane-group width when it is 64 (a whole wave per row: q/k/v,
 // o-proj and LM head of the configs), known at compile time so that the
 // walk's lane map and row sums fold; 0: a.G.
-// STAGE (q8_0 rows of 64-lane groups whose limb buffer is one xq_at block
+// XM: X_LIMBS the lanes read their units' limbs from a.xq; X_BUILD the
+// workgroup builds them in LDS from a.raw; X_STAGE (q8_0 rows of 64-lane groups whose limb buffer is one xq_at block
 // of a multiple of 128 values): every wave reads the whole limb vector, so
 // the workgroup loads it once, 2 UPL 16-byte pieces per thread issued before
 // the weights, and the waves read it from LDS -- a quarter of the limb
 // traffic through the CU's memory pipeline.  Taken for workgroups of many
 // rows (the launcher's choice).
-template <int T, int UPL, int GC, bool STAGE>
+template <int T, int UPL, int GC, int XM>
 __global__ void __launch_bounds__(WG) k_mv_dense(DenseK a)
 {
+    constexpr bool STAGE = XM == X_STAGE;
     const int r_begin = blockIdx.x * a.rpw, r_end = min(a.total, r_begin + a.rpw);
     constexpr int XC = STAGE ? 2 * UPL : 1;
     extern __shared__ __align__(16) uint8_t s_xq[];
@@ -162,6 +216,9 @@ __global__ void __launch_bounds__(WG) k_mv_dense(DenseK a)
 #pragma unroll
         for (int j = 0; j < XC; j++) xc[j] = src[min((int)threadIdx.x + WG * j, nxc - 1)];
     }
+    __shared__ float red[16];
+    XBuild xb;
+    if constexpr (XM == X_BUILD) xb.load(a.raw, ncols);
     unsigned long long best = 0;  // argmax_key of the best row this lane emitted
     // the segments are walked as one stack of rows, so that a workgroup's
     // rows that span two segments stream in one pass
@@ -179,6 +236,10 @@ __global__ void __launch_bounds__(WG) k_mv_dense(DenseK a)
                 if ((int)threadIdx.x + WG * j < nxc) ((styx_u4 *)s_xq)[threadIdx.x + WG * j] = xc[j];
             __syncthreads();
             XFrom<T, UPL>{xq_at(s_xq, ncols)}(x, lu);
+        } else if constexpr (XM == X_BUILD) {
+            const Xq q = xq_at(s_xq, ncols);
+            xb.limbs(a.raw, ncols, q, red);
+            XFrom<T, UPL>{q}(x, lu);
         } else {
             XFrom<T, UPL>{a.xq}(x, lu);
         }
@@ -242,6 +303,36 @@ __global__ void __launch_bounds__(WG) k_mv_dense(DenseK a)
     }
 }
 
+// The launch of a dense walk: XM as the caller chose it for q8_0 64-lane
+// walks (X_STAGE is instantiated for those only).
+template <int T, bool BUILD> static void dense_go(hipStream_t st, const Geo &g, dim3 grid, size_t lds, bool stage, const DenseK &a)
+{
+    constexpr int XM = BUILD ? X_BUILD : X_LIMBS;
+    upl_dispatch<T>(g.UPL, [&](auto u) {
+        constexpr int U = decltype(u)::value;
+        if constexpr (T == T_Q8_0 && !BUILD)
+            if (g.G == 64 && stage) {
+                hipLaunchKernelGGL((k_mv_dense<T, U, 64, X_STAGE>), grid, dim3(WG), lds, st, a);
+                return;
+            }
+        if (g.G == 64)
+            hipLaunchKernelGGL((k_mv_dense<T, U, 64, XM>), grid, dim3(WG), lds, st, a);
+        else
+            hipLaunchKernelGGL((k_mv_dense<T, U, 0, XM>), grid, dim3(WG), lds, st, a);
+    });
+}
+template <bool BUILD> static hipError_t dense_type(hipStream_t st, int t, const Geo &g, dim3 grid, size_t lds, bool stage, const DenseK &a)
+{
+    switch (t) {
+    case T_Q8_0: dense_go<T_Q8_0, BUILD>(st, g, grid, lds, stage, a); break;
+    case T_Q4_K: dense_go<T_Q4_K, BUILD>(st, g, grid, lds, stage, a); break;
+    case T_Q5_K: dense_go<T_Q5_K, BUILD>(st, g, grid, lds, stage, a); break;
+    case T_Q6_K: dense_go<T_Q6_K, BUILD>(st, g, grid, lds, stage, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_dense(hipStream_t st, int t, int ncols, const DenseSeg *segs, int nseg,
                         const Xq &xq, int add, const NormScale *ns, unsigned long long *amax)
 {
@@ -278,24 +369,41 @@ hipError_t launch_dense(hipStream_t st, int t, int ncols, const DenseSeg *segs, 
     const bool stage = ((g.UPL == 1 && a.rpw >= 32) || g.UPL == 4) && ncols % 128 == 0 && ((uintptr_t)xq.A & 15) == 0 && xq.B == xc.B &&
                        xq.C == xc.C && xq.sx == xc.sx && xq.s16 == xc.s16;
     const size_t lds_xq = stage ? xq_bytes(ncols) : 0;
-    switch (t) {
-    case T_Q8_0: upl_dispatch<T_Q8_0>(g.UPL, [&](auto u) {
-        constexpr int U = decltype(u)::value;
-        if (g.G == 64 && stage) hipLaunchKernelGGL((k_mv_dense<T_Q8_0, U, 64, true>), grid, dim3(WG), lds_xq, st, a);
-        else if (g.G == 64) hipLaunchKernelGGL((k_mv_dense<T_Q8_0, U, 64, false>), grid, dim3(WG), 0, st, a);
-        else hipLaunchKernelGGL((k_mv_dense<T_Q8_0, U, 0, false>), grid, dim3(WG), 0, st, a); }); break;
-    case T_Q4_K: upl_dispatch<T_Q4_K>(g.UPL, [&](auto u) {
-        if (g.G == 64) hipLaunchKernelGGL((k_mv_dense<T_Q4_K, decltype(u)::value, 64, false>), grid, dim3(WG), 0, st, a);
-        else hipLaunchKernelGGL((k_mv_dense<T_Q4_K, decltype(u)::value, 0, false>), grid, dim3(WG), 0, st, a); }); break;
-    case T_Q5_K: upl_dispatch<T_Q5_K>(g.UPL, [&](auto u) {
-        if (g.G == 64) hipLaunchKernelGGL((k_mv_dense<T_Q5_K, decltype(u)::value, 64, false>), grid, dim3(WG), 0, st, a);
-        else hipLaunchKernelGGL((k_mv_dense<T_Q5_K, decltype(u)::value, 0, false>), grid, dim3(WG), 0, st, a); }); break;
-    case T_Q6_K: upl_dispatch<T_Q6_K>(g.UPL, [&](auto u) {
-        if (g.G == 64) hipLaunchKernelGGL((k_mv_dense<T_Q6_K, decltype(u)::value, 64, false>), grid, dim3(WG), 0, st, a);
-        else hipLaunchKernelGGL((k_mv_dense<T_Q6_K, decltype(u)::value, 0, false>), grid, dim3(WG), 0, st, a); }); break;
-    default: return hipErrorInvalidValue;
+    return dense_type<false>(st, t, g, grid, lds_xq, stage, a);
+}
+
+hipError_t launch_dense_f32(hipStream_t st, int t, const uint8_t *w, int nrows, int ncols,
+                            const float *x, const float *norm_w, float eps, float *y, int add,
+                            const Xq &scratch)
+{
+    const Geo g = pick_geo(t, ncols);
+    if (g.G == 0 || nrows < 1 || ncols < 32 || ncols % 32 || ncols > XQ_MAX) return hipErrorInvalidValue;
+    // The limbs first, by one k_xq, when y is rewritten while other
+    // workgroups would still read x, and for long rows of many-row matrices:
+    // past 2048 columns the vector is read only after the weights are issued
+    // and its limbs cost the weights' registers, which a workgroup of few
+    // rows (up to 4096 rows in all) hides and one of many does not.  Limbs
+    // first -> built here: 512 x 2048 q8_0 with norm 8.0 -> 4.5 us, 151936 x
+    // 2048 q6_K 49.6 -> 45.3, 2048 x 8192 q6_K 12.3 -> 9.5; but 16384 x 8192
+    // q6_K 44.9 -> 49.7, 16384 x 6144 q4_K 23.6 -> 34.6.
+    if (overlap(x, ncols, y, nrows) || overlap(norm_w, ncols, y, nrows) || (ncols > 8 * WG && nrows > 4096)) {
+        hipError_t e = launch_xq(st, x, nullptr, norm_w, eps, ncols, scratch, nullptr);
+        if (e != hipSuccess) return e;
+        DenseSeg s{w, y, nrows};
+        return launch_dense(st, t, ncols, &s, 1, scratch, add);
     }
-    return hipGetLastError();
+    DenseK a{};
+    a.w[0] = w;
+    a.y[0] = y;
+    a.rows[0] = a.total = nrows;
+    a.nseg = 1;
+    a.nb = ncols / blk_elems(t);
+    a.G = g.G;
+    a.UPL = g.UPL;
+    a.add = add;
+    a.raw = XRaw{x, norm_w, eps};
+    a.rpw = rows_per_wg(nrows, g.G, 1024);
+    return dense_type<true>(st, t, g, dim3((nrows + a.rpw - 1) / a.rpw), xq_bytes(ncols), false, a);
 }
 
 __global__ void __launch_bounds__(64) k_topk(const float *logits, int n, int k, int renorm,
@@ -407,6 +515,8 @@ struct GateUpK {
     const int32_t *id_one;
     uint32_t n_slabs;
     float *h;  // k_gate_up_silu: [nslots][F] = silu(gate rows) * up rows
+    XRaw raw;  // k_gate_up<.., true>: the vector (xq unused)
+    int H;
 };
 
 // Slab of matrix m (0 gate, 1 up) for slot s < k from an id row in memory
@@ -426,12 +536,15 @@ __device__ __forceinline__ const uint8_t *gu_slab_of_ids(const GateUpK &a, int m
 
 // Routing first (one trip for the logits, then LDS work), then the slot's
 // weight loads, then the activation limbs.
-template <int T, int UPL>
-__device__ inline void gate_up_body(const GateUpK &a, int m, int s, int32_t *s_ids, float *s_lg)
+template <int T, int UPL, bool BUILD>
+__device__ inline void gate_up_body(const GateUpK &a, int m, int s, int32_t *s_ids, float *s_lg,
+                                    uint8_t *s_xq, float *red)
 {
+    XBuild xb;
+    if constexpr (BUILD) xb.load(a.raw, a.H);
     const uint8_t *slab;
     if (s < a.k) {
-        if (a.route.logits) {
+        if (!BUILD && a.route.logits) {
             uint32_t r3[3];
             const int32_t *ids = route_ids_wg(a.route, s_ids, s_lg);
             route_row(a.route, ids[s], s, r3);
@@ -453,22 +566,30 @@ __device__ inline void gate_up_body(const GateUpK &a, int m, int s, int32_t *s_i
     walk_rows_pipelined<T, UPL, 1>(
         OneMat{mat, a.nb}, a.nb, a.G, r_begin, r_end,
         [&](UX<T>(&x)[UPL], const LaneU<UPL> &lu) {
-            XFrom<T, UPL>{a.xq}(x, lu);
+            if constexpr (BUILD) {
+                const Xq q = xq_at(s_xq, a.H);
+                xb.limbs(a.raw, a.H, q, red);
+                XFrom<T, UPL>{q}(x, lu);
+            } else {
+                XFrom<T, UPL>{a.xq}(x, lu);
+            }
             return true;
         },
         [=](int r, float v) { y[r] = v; });
 }
 
-template <int TG, int TU, int UPL>
+template <int TG, int TU, int UPL, bool BUILD>
 __global__ void __launch_bounds__(WG) k_gate_up(GateUpK a)
 {
     __shared__ int32_t s_ids[IDS_ROW];
-    __shared__ __align__(16) float s_lg[MAX_EXPERTS];
+    __shared__ __align__(16) float s_lg[BUILD ? 4 : MAX_EXPERTS];
+    __shared__ float red[16];
+    extern __shared__ __align__(16) uint8_t s_xq[];
     const int s = blockIdx.y, m = blockIdx.z;
     if (m == 0)
-        gate_up_body<TG, UPL>(a, 0, s, s_ids, s_lg);
+        gate_up_body<TG, UPL, BUILD>(a, 0, s, s_ids, s_lg, s_xq, red);
     else
-        gate_up_body<TU, UPL>(a, 1, s, s_ids, s_lg);
+        gate_up_body<TU, UPL, BUILD>(a, 1, s, s_ids, s_lg, s_xq, red);
 }
 
 // Gate and up rows [r0, r1) of one slot in one workgroup, then
@@ -509,31 +630,50 @@ __global__ void __launch_bounds__(WG) k_gate_up_silu(GateUpK a)
 }
 
 // gate and up share the block size, so one geometry serves both
+template <int TG, int TU>
+static hipError_t gu_go(hipStream_t st, int upl, const GateUpK &a, dim3 grid)
+{
+    upl_dispatch<TG>(upl, [&](auto u) {
+        constexpr int U = decltype(u)::value;
+        if (a.raw.x)
+            hipLaunchKernelGGL((k_gate_up<TG, TU, U, true>), grid, dim3(WG), xq_bytes(a.H), st, a);
+        else
+            hipLaunchKernelGGL((k_gate_up<TG, TU, U, false>), grid, dim3(WG), 0, st, a);
+    });
+    return hipGetLastError();
+}
 template <int TG>
 static hipError_t launch_gu_tu(hipStream_t st, int tu, int upl, const GateUpK &a, dim3 grid)
 {
     if constexpr (TG == T_Q8_0) {
-        if (tu != T_Q8_0) return hipErrorInvalidValue;
-        upl_dispatch<T_Q8_0>(upl, [&](auto u) { hipLaunchKernelGGL((k_gate_up<TG, T_Q8_0, decltype(u)::value>), grid, dim3(WG), 0, st, a); });
+        return tu == T_Q8_0 ? gu_go<TG, T_Q8_0>(st, upl, a, grid) : hipErrorInvalidValue;
     } else {
         switch (tu) {
-        case T_Q4_K: upl_dispatch<T_Q4_K>(upl, [&](auto u) { hipLaunchKernelGGL((k_gate_up<TG, T_Q4_K, decltype(u)::value>), grid, dim3(WG), 0, st, a); }); break;
-        case T_Q5_K: upl_dispatch<T_Q5_K>(upl, [&](auto u) { hipLaunchKernelGGL((k_gate_up<TG, T_Q5_K, decltype(u)::value>), grid, dim3(WG), 0, st, a); }); break;
-        case T_Q6_K: upl_dispatch<T_Q6_K>(upl, [&](auto u) { hipLaunchKernelGGL((k_gate_up<TG, T_Q6_K, decltype(u)::value>), grid, dim3(WG), 0, st, a); }); break;
+        case T_Q4_K: return gu_go<TG, T_Q4_K>(st, upl, a, grid);
+        case T_Q5_K: return gu_go<TG, T_Q5_K>(st, upl, a, grid);
+        case T_Q6_K: return gu_go<TG, T_Q6_K>(st, upl, a, grid);
         default: return hipErrorInvalidValue;
         }
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_moe_gate_up(hipStream_t st, int tg, int tu, const ExpSrc &g, const ExpSrc &u,
                               const int32_t *ids, const Route *route, const Xq &xq, float *gu,
                               int H, int F, int k, const uint8_t *sh_gate, const uint8_t *sh_up,
-                              int filter)
+                              int filter, const float *x)
 {
     const Geo gg = pick_geo(tg, H);
     if (!gg.G || blk_elems(tg) != blk_elems(tu) || k < 1 || k > MAX_TOPK || !xq.A)
         return hipErrorInvalidValue;
+    if (x && (route || H > XQ_MAX)) return hipErrorInvalidValue;
+    // limbs built by the workgroups (30B-A3B experts: one launch less, 3.4 us)
+    // unless the outputs rewrite x while other workgroups still read it, or
+    // H is past the 4096 columns this was measured to pay at
+    if (x && (H > 4096 || overlap(x, H, gu, (int64_t)2 * k * F))) {
+        hipError_t e = launch_xq(st, x, nullptr, nullptr, 0.0f, H, xq, nullptr);
+        if (e != hipSuccess) return e;
+        x = nullptr;
+    }
     if (route && (route->E < k || route->E > MAX_EXPERTS || route->E % 16 || route->k != k))
         return hipErrorInvalidValue;
     if (!route && !ids) return hipErrorInvalidValue;
@@ -552,6 +692,8 @@ hipError_t launch_moe_gate_up(hipStream_t st, int tg, int tu, const ExpSrc &g, c
     a.k = k;
     a.filter = filter;
     a.nb = H / blk_elems(tg);
+    a.raw.x = x;
+    a.H = H;
     // ~1024 workgroups in total over the 2*k slot matrices
     a.rpw = rows_per_wg(2 * a.nslots * F, gg.G, 1024);
     const dim3 grid((F + a.rpw - 1) / a.rpw, a.nslots, 2);

@@ -154,3 +154,72 @@ def test_attn_in_async_and_plain_batches(gpu):
             assert rel_l2(binds[3].download(np.float32), ref) < 2e-6
     for o in (ab, mb, k, t):
         o.free()
+
+
+# op matvec: limbs built by the workgroups (up to 2048 columns, or few rows)
+# or by a launch in front (long rows of many rows, outputs over the input)
+@pytest.mark.parametrize("t,rows,cols", [(8, 40, 32), (8, 33, 2048), (8, 16, 2112), (12, 64, 4096),
+                                         (14, 4096, 3072), (14, 4098, 3072), (13, 24, 8192)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_op_matvec_against_f64(gpu, t, rows, cols, norm):
+    import ctypes as C
+    from styx_amd import _lib as L
+    from styx_amd.runtime import to_split
+    a = weights(t, rows, cols, rows)
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal(cols).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+    w = to_split(gpu, t, gpu.from_numpy(a), rows, cols)
+    bx, bn, by = f32buf(gpu, x), f32buf(gpu, nw), gpu.zeros(rows * 4)
+    L.check(gpu.lib.styx_op_matvec(gpu.h, t, w.ptr, rows, cols, bx.ptr, bn.ptr if norm else None,
+                                   C.c_float(1e-6), by.ptr, 0))
+    gpu.sync()
+    xd = x.astype(np.float64)
+    xn = (xd / np.sqrt((xd ** 2).mean() + 1e-6) * nw) if norm else xd
+    y = O.matvec_f64(t, a, rows, cols, xn.astype(np.float32))
+    bound = sum_bound(t, a, rows, cols, xn.astype(np.float32)) + 1e-6 * np.abs(y).max()
+    assert (np.abs(by.download(np.float32, rows) - y) <= bound).all()
+
+
+def test_op_matvec_in_place(gpu):
+    """y over x: the product of the old x, as with the limbs formed first."""
+    import ctypes as C
+    from styx_amd import _lib as L
+    from styx_amd.runtime import to_split
+    t, n = 8, 2048
+    a = weights(t, n, n, 77)
+    x = np.random.default_rng(6).standard_normal(n).astype(np.float32)
+    w = to_split(gpu, t, gpu.from_numpy(a), n, n)
+    apart, inplace, by = f32buf(gpu, x), f32buf(gpu, x), gpu.zeros(n * 4)
+    f = gpu.lib.styx_op_matvec
+    L.check(f(gpu.h, t, w.ptr, n, n, apart.ptr, None, C.c_float(0.0), by.ptr, 0))
+    L.check(f(gpu.h, t, w.ptr, n, n, inplace.ptr, None, C.c_float(0.0), inplace.ptr, 0))
+    gpu.sync()
+    assert np.array_equal(by.download(np.float32), inplace.download(np.float32))
+
+
+@pytest.mark.parametrize("E,k", [(16, 4), (64, 16), (65, 8), (200, 10), (512, 10)])
+def test_topk_ties_and_unordered_entries(gpu, E, k):
+    """Ties keep the lower index; -inf and NaN entries are never picked."""
+    lg = np.random.default_rng(E).integers(-3, 4, E).astype(np.float32)
+    lg[1], lg[5] = -np.inf, -0.0
+    bw, bi = gpu.zeros(64), gpu.from_numpy(np.full(64, -7, np.int32))
+    ident = gpu.from_numpy(np.arange(E, dtype=np.uint32))
+    skip = gpu.from_numpy(np.full(E, SKIP, np.uint32))
+
+    def go(v):
+        run(gpu, "topk_softmax_f32", [f32buf(gpu, v), bw, bi, ident, skip], struct.pack("<3I", E, k, 1),
+            (1, 1, 1))
+        return bi.download(np.int32, 16 + k), bw.download(np.float32, k)
+    ids, w = go(lg)
+    w_ref, ids_ref = O.topk_softmax(lg, k, True, None, None)
+    assert np.array_equal(ids[:k], ids_ref[:k]) and np.array_equal(ids[16:16 + k], ids_ref[:k])
+    assert rel_l2(w, w_ref) < 1e-6
+    nan = lg.copy()
+    nan[ids[0]] = np.nan
+    got, _ = go(nan)
+    order = [e for e in sorted(range(E), key=lambda e: (-lg[e], e)) if e != ids[0]][:k]
+    assert got[:k].tolist() == order
+
+
+SKIP = 0xFFFFFFFF
