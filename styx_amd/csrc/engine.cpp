@@ -196,7 +196,12 @@ struct styx_moe {
         int4 *tiles;
         int *ntiles;
         void *vec_h, *vec_o, *vec_f;  // pieces of H-, q_dim- and F-wide rows
+        // experts in host memory: the cold ones of a layer, and a buffer that
+        // one of its tensors' cold slabs pass through (those that fit)
+        int *cold_slot, *cold_list, *ncold;
+        uint8_t *stage;
     } pb{};
+    static constexpr int64_t PB_STAGE = 64ll << 20;
     uint64_t repin_swaps = 0;
     std::vector<void *> dev_allocs, host_allocs;
     // timing
@@ -1040,6 +1045,10 @@ int styx_moe::prompt_workspace()
         put(&w.ntiles, 4);
         put((char **)&w.vec_h, prompt_vec_bytes(T, H));
         put((char **)&w.vec_o, prompt_vec_bytes(T, (int)qd));
+        put(&w.cold_slot, 4 * (size_t)E);
+        put(&w.cold_list, 4 * (size_t)E);
+        put(&w.ncold, 4);
+        put(&w.stage, any_host ? (size_t)PB_STAGE : 0);
         put((char **)&w.vec_f, std::max(prompt_vec_bytes(P, F), Fsh ? prompt_vec_bytes(T, Fsh) : 0));
     };
     lay(pb);
@@ -1058,6 +1067,7 @@ int styx_moe::prompt_workspace()
     at(&pb.logits), at(&pb.wts), at(&pb.g), at(&pb.u), at(&pb.y), at(&pb.sh_y), at(&pb.gate);
     at(&pb.ids), at(&pb.order), at(&pb.inv), at(&pb.tiles), at(&pb.ntiles);
     at((char **)&pb.vec_h), at((char **)&pb.vec_o), at((char **)&pb.vec_f);
+    at(&pb.cold_slot), at(&pb.cold_list), at(&pb.ncold), at(&pb.stage);
     pb_t = T;
     return STYX_OK;
 }
@@ -1166,6 +1176,12 @@ int styx_moe::prompt_batch(const uint32_t *tok, int n)
             rt.k = K;
             rt.renorm = norm_topk;
             rt.tile_tokens = te;
+            if (ly.host_experts) {
+                rt.remap = ly.remap_dev;
+                rt.cold_slot = pb.cold_slot;
+                rt.cold_list = pb.cold_list;
+                rt.ncold = pb.ncold;
+            }
             CK(launch_prompt_route(st, rt));
             if (sh) {
                 const PromptVec vs = prompt_vec_at(pb.vec_f, T, Fsh);
@@ -1188,11 +1204,22 @@ int styx_moe::prompt_batch(const uint32_t *tok, int n)
                 g.xdiv = K;
                 int type = -1;
                 for (auto &m : ms) {
-                    if (g.nseg && m.first->type != type) {
+                    // (the staging buffer holds one tensor's slabs at a time)
+                    if (g.nseg && (m.first->type != type || ly.host_experts)) {
                         if (hipError_t e = launch_prompt_gemm(st, type, g)) return e;
                         g.nseg = 0;
                     }
                     type = m.first->type;
+                    if (ly.host_experts) {
+                        g.stage = pb.stage;
+                        g.cold_slot = pb.cold_slot;
+                        g.stage_slots = (int)std::min<int64_t>(E, PB_STAGE / m.first->slab);
+                        const int most = std::min(g.stage_slots, P);  // as many experts as pairs
+                        if (most > 0)
+                            if (hipError_t e = launch_prompt_stage(st, pb.cold_list, pb.ncold, m.first->host_dev,
+                                                                   m.first->slab, pb.stage, most))
+                                return e;
+                    }
                     ExpSrc &s = g.src[g.nseg];
                     s = ExpSrc{};
                     s.hot = ly.host_experts ? m.first->hot : m.first->dev;

@@ -384,6 +384,9 @@ struct PromptGemm {
     int max_tiles;
     ExpSrc src[3];         // per segment, with tiles
     const uint32_t *remap; // expert -> hot slot or SKIP (read from gtt); null: itself
+    const uint8_t *stage;  // slabs of the cold experts of slot < stage_slots, or null
+    const int *cold_slot;
+    int stage_slots;
     const int *order;      // activation row of a position: order[pos] / xdiv; null: pos
     int xdiv;
     int rt0[3], nrt, ntt;  // filled by the launch
@@ -411,6 +414,10 @@ struct PromptRoute {
     int4 *tiles;
     int *ntiles;
     int T, E, H, k, renorm, tile_tokens;
+    // experts in host memory (remap null: none): the met ones that are not
+    // hot, as a list and as each one's place there
+    const uint32_t *remap;
+    int *cold_slot, *cold_list, *ncold;
 };
 
 hipError_t launch_prompt_embed(hipStream_t st, int t, const uint8_t *w, int64_t nrows, int ncols,
@@ -419,6 +426,9 @@ hipError_t launch_prompt_pack(hipStream_t st, int mode, const PromptPack &a, int
 hipError_t launch_prompt_gemm(hipStream_t st, int t, PromptGemm a);
 hipError_t launch_prompt_rope(hipStream_t st, const PromptAttn &a);
 hipError_t launch_prompt_attn(hipStream_t st, const PromptAttn &a);
+// The first `slots` cold experts' slabs of one tensor to dst, slab bytes apart.
+hipError_t launch_prompt_stage(hipStream_t st, const int *list, const int *ncold, const uint8_t *src,
+                               int64_t slab, uint8_t *dst, int slots);
 // Router logits, top-k ids and weights, and the pairs grouped by expert.
 hipError_t launch_prompt_route(hipStream_t st, const PromptRoute &a);
 

@@ -109,14 +109,25 @@ template <int MODE> __global__ void __launch_bounds__(PWG) k_prompt_pack(PromptP
             for (int j = 0; j < 4; j++) v[j] = v[j] / (1.0f + expf(-v[j])) * u[j];
         }
         if constexpr (MODE == PACK_COMBINE) {
+            // eight slots' rows in flight at once; an absent slot reads row 0
+            // and adds nothing
             f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int s = 0; s < a.k; s++) {
-                const int p = a.inv[row * a.k + s];
-                if (p < 0) continue;
-                const float w = a.wts[row * MAX_TOPK + s];
-                const f4 y = *(const f4 *)(a.y + (int64_t)p * a.n + i);
+            for (int s0 = 0; s0 < a.k; s0 += 8) {
+                f4 y[8];
+                float w[8];
+                bool on[8];
 #pragma unroll
-                for (int j = 0; j < 4; j++) acc[j] += w * y[j];
+                for (int s = 0; s < 8; s++) {
+                    const int p = s0 + s < a.k ? a.inv[row * a.k + s0 + s] : -1;
+                    on[s] = p >= 0;
+                    w[s] = s0 + s < a.k ? a.wts[row * MAX_TOPK + s0 + s] : 0.0f;
+                    y[s] = *(const f4 *)(a.y + (int64_t)max(p, 0) * a.n + i);
+                }
+#pragma unroll
+                for (int s = 0; s < 8; s++)
+                    if (on[s])
+#pragma unroll
+                        for (int j = 0; j < 4; j++) acc[j] += w[s] * y[s][j];
             }
             v += acc;
             if (a.y_sh) {
@@ -527,7 +538,7 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
 }
 
 // Y[pos][r] = sum_c W[r][c] x[row(pos)][c] for a tile of 16 TT positions and
-// 64 NG rows per workgroup (16 NG rows per wave), the activation pieces of a
+// 16 NG rows per wave of a workgroup of NW, the activation pieces of a
 // step in LDS (shared by the waves), each wave's weights in its registers
 // one step ahead.  With tiles, tile i holds positions [start, start + count)
 // of one expert (its slab) and row(pos) = order[pos] / xdiv or pos; without,
@@ -537,14 +548,15 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
 // (three or four f16 products per value) beyond; 16 TT = 32 tokens keeps an
 // expert's tile near the 24 tokens an expert meets in 384-token prompts at
 // k / E = 8 / 128 and two workgroups on a CU.  At 383 tokens of the 30B-A3B
-// shape: q/k/v (5120 x 2048 q8_0) 52 us, gate (q4_K) 86, up (q5_K) 111, down
-// (q6_K) 96 us for 417 MB of slabs; a 384-token prompt through two such
-// layers took 51.7 ms token by token and takes 1.1 ms (with two generated
-// tokens), the batch itself 0.56 ms.
-template <int T, bool D8, int TT, int NG>
-__global__ void __launch_bounds__(PWG, 2) k_prompt_gemm(PromptGemm a)
+// shape: q/k/v (5120 x 2048 q8_0) 48 us, gate (q4_K) 87, up (q5_K) 111, down
+// (q6_K) 90 us for 417 MB of slabs; a 384-token prompt through two such
+// layers took 51.7 ms token by token and takes 1.05 ms (with two generated
+// tokens), the batch itself 0.53 ms.
+template <int T, bool D8, int TT, int NG, int NW>
+__global__ void __launch_bounds__(64 * NW, 2) k_prompt_gemm(PromptGemm a)
 {
-    constexpr int TM = 16 * TT, XR = 2 * TT;
+    constexpr int TM = 16 * TT, XT = 2 * NW, XR = TM / XT;  // rows staged per pass, passes
+    static_assert(TM % XT == 0, "whole passes");
     __shared__ __align__(16) uint8_t s_x[3 * TM * XROW];
     __shared__ __align__(16) uint8_t s_sum[TM * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
@@ -575,7 +587,12 @@ __global__ void __launch_bounds__(PWG, 2) k_prompt_gemm(PromptGemm a)
         count = ti.z;
         const uint32_t h = a.remap ? a.remap[ti.x] : (uint32_t)ti.x;
         const ExpSrc &e = a.src[seg];
-        base = h != SKIP ? e.hot + (int64_t)h * e.hot_slab : e.gtt + (int64_t)ti.x * e.gtt_slab;
+        if (h != SKIP)
+            base = e.hot + (int64_t)h * e.hot_slab;
+        else if (const int c = a.stage ? a.cold_slot[ti.x] : a.stage_slots; c < a.stage_slots)
+            base = a.stage + (int64_t)c * e.gtt_slab;
+        else
+            base = e.gtt + (int64_t)ti.x * e.gtt_slab;
     }
     auto xrow = [&](int i) {  // activation row of position start + i (clamped to the tile)
         const int p = start + min(i, count - 1);
@@ -587,16 +604,16 @@ __global__ void __launch_bounds__(PWG, 2) k_prompt_gemm(PromptGemm a)
     const Buf m(base, nblk * blk_bytes(T));
     const Reg ro{(uint32_t)region_off(sl, 1, nblk), (uint32_t)region_off(sl, 2, nblk),
                  (uint32_t)region_off(sl, 3, nblk)};
-    const int r0 = rt * 64 * NG + wave * 16 * NG;
+    const int r0 = (rt * NW + wave) * 16 * NG;
     PW<T, D8> w[NG];
     auto wload = [&](int c) {
 #pragma unroll
         for (int r = 0; r < NG; r++) w[r].load(m, ro, min(r0 + 16 * r + n, rows - 1), nb, c, g);
     };
-    // this thread's 16-byte columns of 2 TT rows of each piece
+    // this thread's 16-byte columns of XR rows of each piece
     uint32_t xo[XR];
 #pragma unroll
-    for (int i = 0; i < XR; i++) xo[i] = (uint32_t)xrow((tid >> 5) + 8 * i) * a.x.np * 2 + (tid & 31) * 16;
+    for (int i = 0; i < XR; i++) xo[i] = (uint32_t)xrow((tid >> 5) + XT * i) * a.x.np * 2 + (tid & 31) * 16;
     const int64_t plane = a.x.rows * (int64_t)a.x.np * 2;
     const Buf xb[3] = {{a.x.p, plane}, {(const uint8_t *)a.x.p + plane, plane}, {(const uint8_t *)a.x.p + 2 * plane, plane}};
     const Buf sb(a.x.sums, a.x.rows * nc * 64);
@@ -615,24 +632,26 @@ __global__ void __launch_bounds__(PWG, 2) k_prompt_gemm(PromptGemm a)
     for (int r = 0; r < NG; r++)
 #pragma unroll
         for (int t = 0; t < TT; t++) acc[r][t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    wload(0);
     xload(0);
+    wload(0);
     for (int c = 0; c < nc; c++) {
         __syncthreads();
 #pragma unroll
         for (int p = 0; p < 3; p++)
 #pragma unroll
             for (int i = 0; i < XR; i++)
-                *(styx_u4 *)(s_x + (p * TM + (tid >> 5) + 8 * i) * XROW + (tid & 31) * 16) = xr[p * XR + i];
+                *(styx_u4 *)(s_x + (p * TM + (tid >> 5) + XT * i) * XROW + (tid & 31) * 16) = xr[p * XR + i];
         if (T == T_Q4_K || T == T_Q5_K)
             if (tid < TM * 4) *(styx_u4 *)(s_sum + tid * 16) = sr;
         __syncthreads();
         PW<T, D8> wc[NG];
 #pragma unroll
         for (int r = 0; r < NG; r++) wc[r] = w[r];
+        // (the activations first: loads return in order, and the LDS stores
+        // of the next step then leave its weights in flight)
         if (c + 1 < nc) {
-            wload(c + 1);
             xload(c + 1);
+            wload(c + 1);
         }
         gemm_step<T, D8, NG, TT>(
             wc,
@@ -742,32 +761,36 @@ template <int T, bool D8> static hipError_t gemm_few(hipStream_t st, PromptGemm 
     return hipGetLastError();
 }
 
-template <int T, bool D8, int TT, int NG> static hipError_t gemm_go(hipStream_t st, PromptGemm &a)
+template <int T, bool D8, int TT, int NG, int NW> static hipError_t gemm_go(hipStream_t st, PromptGemm &a)
 {
     a.nrt = 0;
     for (int s = 0; s < a.nseg; s++) {
         a.rt0[s] = a.nrt;
-        a.nrt += (a.rows[s] + 64 * NG - 1) / (64 * NG);
+        a.nrt += (a.rows[s] + 16 * NW * NG - 1) / (16 * NW * NG);
     }
     a.ntt = (a.T + 16 * TT - 1) / (16 * TT);
     const int64_t n = a.tiles ? (int64_t)((a.max_tiles + 7) / 8 * 8) * a.nrt
                               : (int64_t)((a.nrt + 7) / 8 * 8) * a.ntt;
     if (n > 0x7FFFFFFF) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_prompt_gemm<T, D8, TT, NG>), dim3((unsigned)n), dim3(PWG), 0, st, a);
+    hipLaunchKernelGGL((k_prompt_gemm<T, D8, TT, NG, NW>), dim3((unsigned)n), dim3(64 * NW), 0, st, a);
     return hipGetLastError();
 }
 
 template <int T, bool D8 = true> static hipError_t gemm_t(hipStream_t st, PromptGemm &a)
 {
-    // 32 positions a tile unless 16 hold them all; two row tiles per wave
-    // (each activation operand read from LDS serves both) unless that would
-    // leave CUs without a workgroup
+    // 32 positions a tile unless 16 hold them all; eight waves of 16 rows
+    // unless that would leave CUs without a workgroup, then four.  Four waves
+    // of two row tiles each (half the LDS reads per product, 220 registers)
+    // measured the same but for q5_K, whose unpacking takes the most
+    // registers: 111 against 119 us for the up slabs of 383 tokens.
     const int64_t rows = (int64_t)a.rows[0] + (a.nseg > 1 ? a.rows[1] : 0) + (a.nseg > 2 ? a.rows[2] : 0);
     if (!a.tiles && a.T <= 32) return gemm_few<T, D8>(st, a);
     const int tm = a.tile_tokens;
-    const int64_t wg2 = (rows + 127) / 128 * (a.tiles ? a.max_tiles : (a.T + tm - 1) / tm);
-    if (tm == 16) return wg2 < 256 ? gemm_go<T, D8, 1, 1>(st, a) : gemm_go<T, D8, 1, 2>(st, a);
-    return wg2 < 256 ? gemm_go<T, D8, 2, 1>(st, a) : gemm_go<T, D8, 2, 2>(st, a);
+    const int64_t wg = (rows + 127) / 128 * (a.tiles ? a.max_tiles : (a.T + tm - 1) / tm);
+    if (tm == 16) return wg < 256 ? gemm_go<T, D8, 1, 1, 4>(st, a) : gemm_go<T, D8, 1, 1, 8>(st, a);
+    if (wg < 256) return gemm_go<T, D8, 2, 1, 4>(st, a);
+    if constexpr (T == T_Q5_K) return gemm_go<T, D8, 2, 2, 4>(st, a);
+    return gemm_go<T, D8, 2, 1, 8>(st, a);
 }
 
 hipError_t launch_prompt_gemm(hipStream_t st, int t, PromptGemm a)
@@ -886,6 +909,7 @@ __global__ void __launch_bounds__(PWG) k_prompt_router(const float *xn, const fl
     const float *wp = W + (int64_t)min(e0 + n, E - 1) * H + wave * q + 4 * g;
     const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     f4 acc[4] = {zero, zero, zero, zero};
+#pragma unroll 4
     for (int i = 0; i < q; i += 16) {
         const f4 x = *(const f4 *)(xp + i), w = *(const f4 *)(wp + i);
 #pragma unroll
@@ -914,9 +938,10 @@ __global__ void __launch_bounds__(64) k_prompt_topk(const float *logits, int E, 
 constexpr int PLAN_WG = 1024;
 __global__ void __launch_bounds__(PLAN_WG) k_prompt_plan(const int32_t *ids, int T, int k, int E,
                                                          int tm, int *order, int *inv, int4 *tiles,
-                                                         int *ntiles)
+                                                         int *ntiles, const uint32_t *remap,
+                                                         int *cold_slot, int *cold_list, int *ncold)
 {
-    __shared__ int cnt[MAX_EXPERTS], off[MAX_EXPERTS], til[MAX_EXPERTS];
+    __shared__ int cnt[MAX_EXPERTS], off[MAX_EXPERTS], til[MAX_EXPERTS], cold[MAX_EXPERTS];
     const int tid = threadIdx.x;
     if (tid < MAX_EXPERTS) cnt[tid] = 0;
     __syncthreads();
@@ -925,20 +950,27 @@ __global__ void __launch_bounds__(PLAN_WG) k_prompt_plan(const int32_t *ids, int
         if (e < (uint32_t)E) atomicAdd(&cnt[e], 1);
     }
     __syncthreads();
-    // inclusive scans of the counts and of the tiles they make
-    int c = 0, t = 0;
+    // inclusive scans of the counts, of the tiles they make and of the met
+    // experts that are not in HBM
+    int c = 0, t = 0, host = 0;
     if (tid < MAX_EXPERTS) {
         off[tid] = c = cnt[tid];
         til[tid] = t = (c + tm - 1) / tm;
+        cold[tid] = host = remap && c > 0 && remap[tid] == SKIP;
     }
     __syncthreads();
     for (int d = 1; d < MAX_EXPERTS; d *= 2) {
-        int a = 0, b = 0;
-        if (tid < MAX_EXPERTS && tid >= d) a = off[tid - d], b = til[tid - d];
+        int a = 0, b = 0, h = 0;
+        if (tid < MAX_EXPERTS && tid >= d) a = off[tid - d], b = til[tid - d], h = cold[tid - d];
         __syncthreads();
-        if (tid < MAX_EXPERTS) off[tid] += a, til[tid] += b;
+        if (tid < MAX_EXPERTS) off[tid] += a, til[tid] += b, cold[tid] += h;
         __syncthreads();
     }
+    if (host) {
+        cold_slot[tid] = cold[tid] - 1;
+        cold_list[cold[tid] - 1] = tid;
+    }
+    if (remap && tid == 0) *ncold = cold[MAX_EXPERTS - 1];
     if (tid < MAX_EXPERTS) {
         const int o = off[tid] - c, i0 = til[tid] - t;
         for (int i = 0; i < t; i++) tiles[i0 + i] = make_int4(tid, o + i * tm, min(tm, c - i * tm), 0);
@@ -957,6 +989,38 @@ __global__ void __launch_bounds__(PLAN_WG) k_prompt_plan(const int32_t *ids, int
     }
 }
 
+// Slabs of the first `slots` cold experts from pinned host memory to the
+// staging buffer: blockIdx.y the slot, 64 KiB per workgroup, four 16-byte
+// loads in flight per thread.  The GEMM's own loads of host memory (64-byte
+// pieces of 16 rows) reach about half the link's rate, these 52 GB/s: a
+// 96-token prompt with half of the experts cold (about 55 slabs of each
+// matrix) 6.7 -> 4.0 ms.
+constexpr int64_t STAGE_CHUNK = 64 * 1024;
+__global__ void __launch_bounds__(PWG) k_prompt_stage(const int *list, const int *ncold, const uint8_t *src,
+                                                      int64_t slab, uint8_t *dst)
+{
+    const int s = blockIdx.y;
+    if (s >= *ncold) return;
+    const styx_u4 *p = (const styx_u4 *)(src + (int64_t)list[s] * slab);
+    styx_u4 *q = (styx_u4 *)(dst + (int64_t)s * slab);
+    const int64_t c0 = blockIdx.x * (STAGE_CHUNK / 16), c1 = min(slab / 16, c0 + STAGE_CHUNK / 16);
+    int64_t i = c0 + threadIdx.x;
+    for (; i + 3 * PWG < c1; i += 4 * PWG) {
+        const styx_u4 a = p[i], b = p[i + PWG], c = p[i + 2 * PWG], d = p[i + 3 * PWG];
+        q[i] = a, q[i + PWG] = b, q[i + 2 * PWG] = c, q[i + 3 * PWG] = d;
+    }
+    for (; i < c1; i += PWG) q[i] = p[i];
+}
+
+hipError_t launch_prompt_stage(hipStream_t st, const int *list, const int *ncold, const uint8_t *src,
+                               int64_t slab, uint8_t *dst, int slots)
+{
+    if (slab < 16 || slab % 16 || slots < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_prompt_stage, dim3((unsigned)((slab + STAGE_CHUNK - 1) / STAGE_CHUNK), slots),
+                       dim3(PWG), 0, st, list, ncold, src, slab, dst);
+    return hipGetLastError();
+}
+
 hipError_t launch_prompt_route(hipStream_t st, const PromptRoute &a)
 {
     if (a.T < 1 || a.E < a.k || a.E > MAX_EXPERTS || a.k < 1 || a.k > MAX_TOPK || a.H % 64)
@@ -966,7 +1030,7 @@ hipError_t launch_prompt_route(hipStream_t st, const PromptRoute &a)
     hipLaunchKernelGGL(k_prompt_topk, dim3(a.T), dim3(64), 0, st, a.logits, a.E, a.k, a.renorm, a.wts,
                        a.ids);
     hipLaunchKernelGGL(k_prompt_plan, dim3(1), dim3(PLAN_WG), 0, st, a.ids, a.T, a.k, a.E, a.tile_tokens,
-                       a.order, a.inv, a.tiles, a.ntiles);
+                       a.order, a.inv, a.tiles, a.ntiles, a.remap, a.cold_slot, a.cold_list, a.ncold);
     return hipGetLastError();
 }
 
