@@ -2163,11 +2163,12 @@ int styx_moe_generate(styx_moe *m, const uint32_t *prompt, int n_prompt, int n_p
     using clk = std::chrono::steady_clock;
     const auto t0 = clk::now();
     // every token but the last in batches, unless the host works between
-    // tokens (repinning counts each token's experts, timing each launch) or
-    // a token is out of range: forward_token reports that one, after the
-    // tokens before it as ever
+    // tokens (repinning counts each token's experts, timing each launch),
+    // the rows do not fit a pack workgroup's LDS, or a token is out of range:
+    // forward_token reports that one, after the tokens before it as ever
     int i = 0;
-    if (n_prompt > PROMPT_MIN_T && m->broken.empty() && !m->opts.time_kernels &&
+    const int widest = std::max(std::max(m->H, m->nh * m->hd), std::max(m->F, m->Fsh));
+    if (n_prompt > PROMPT_MIN_T && widest <= PROMPT_MAX_N && m->broken.empty() && !m->opts.time_kernels &&
         !(m->opts.repin_interval > 0 && m->any_host)) {
         int nb = 0;
         while (nb < n_prompt - 1 && prompt[nb] < (uint32_t)m->V) nb++;

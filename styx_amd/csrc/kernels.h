@@ -320,7 +320,8 @@ hipError_t launch_read_probe(hipStream_t st, const void *p, int64_t bytes, uint3
                              int grid);
 
 // ---- prompt batches (prompt.hip) -------------------------------------------
-constexpr int PROMPT_MAX_T = 512;  // most tokens of one batch
+constexpr int PROMPT_MAX_T = 512;    // most tokens of one batch
+constexpr int PROMPT_MAX_N = 15360;  // longest activation row (60 KiB of LDS)
 
 // Activation rows as three f16 pieces of x 2^e, [3][rows][np] (np: n rounded
 // up to whole 256-value steps, zeros past n), the sums of each run of 32

@@ -214,7 +214,7 @@ template <int MODE> __global__ void __launch_bounds__(PWG) k_prompt_pack(PromptP
 
 hipError_t launch_prompt_pack(hipStream_t st, int mode, const PromptPack &a, int rows)
 {
-    if (rows < 1 || a.n < 32 || a.n % 32 || a.n > XQ_MAX || a.v.n != a.n || rows > a.v.rows)
+    if (rows < 1 || a.n < 32 || a.n % 32 || a.n > PROMPT_MAX_N || a.v.n != a.n || rows > a.v.rows)
         return hipErrorInvalidValue;
     const dim3 g(rows), b(PWG);
     const size_t lds = (size_t)a.n * 4;
