@@ -132,7 +132,8 @@ struct styx_moe {
     uint32_t *d_tok = nullptr, *hist = nullptr;
     // running argmax of the LM head (argmax_key), cleared by its reader
     unsigned long long *am_word = nullptr;
-    uint32_t *h_stage = nullptr;  // pinned: tok, pos
+    uint32_t *h_stage = nullptr;  // pinned: [4] the abort flag, [5] the token, of the last read-out
+    uint2 *h_stage_dev = nullptr; // device address of h_stage[4]
     // KV
     float *kpool = nullptr, *vpool = nullptr;
     // pages hold each kv head's rows together ([nkv][page_tokens][hd]): an
@@ -361,6 +362,9 @@ int styx_moe::setup_runtime()
     if (int r = alloc_host(&hs, 64)) return r;
     h_stage = (uint32_t *)hs;
     std::memset(h_stage, 0, 64);
+    void *hd_stage = nullptr;
+    STYX_HIP(hipHostGetDevicePointer(&hd_stage, hs, 0));
+    h_stage_dev = (uint2 *)((uint32_t *)hd_stage + 4);
     // paged KV: pool sized for n_ctx on every layer, pages handed out lazily
     pages_per_layer = (n_ctx + KV_PAGE_TOKENS - 1) / KV_PAGE_TOKENS;
     const size_t pool = (size_t)L * pages_per_layer * KV_PAGE_TOKENS * kv_dim;
@@ -596,8 +600,9 @@ int styx_moe::size_moe_block()
 
 // A fused MoE launch whose wait ran out sets the abort flag; the model's
 // results are then invalid and it stays in error until reloaded.  The flag
-// is copied into the pinned stage (h_stage[4]) ahead of the caller's stream
-// synchronisation (queue_abort_read), then checked here.
+// reaches the pinned stage (h_stage[4]) with every token's read-out
+// (k_argmax_word; queue_abort_read where no token is read out) ahead of the
+// caller's stream synchronisation, then is checked here.
 void styx_moe::queue_abort_read()
 {
     if (mb_abort && !opts.no_fuse)
@@ -961,7 +966,7 @@ int styx_moe::enqueue_token(bool gen, int mode)
     if (want("lm_head")) CK(launch_dense(st, head.type, H, &sh, 1, xq_a, 0, &ns_a, am_word));
     tend(e0, "lm_head", (double)head.bytes() + xq_bytes(H) + 4.0 * V);
     e0 = tstart();
-    if (want("argmax")) CK(launch_argmax_word(st, am_word, d_tok, d_pos, gen ? 1 : 0, hist));
+    if (want("argmax")) CK(launch_argmax_word(st, am_word, d_tok, d_pos, gen ? 1 : 0, hist, mb_abort, h_stage_dev));
     tend(e0, "argmax", 8.0);
     return STYX_OK;
 }
@@ -2056,25 +2061,19 @@ int styx_moe_forward_token(styx_moe *m, uint32_t token, float *logits_out)
     if (m->n_past > 0)
         if (int r = m->maybe_repin()) return r;
     if (int r = m->ensure_pages(m->n_past)) return r;
-    m->h_stage[0] = token;
-    m->h_stage[1] = (uint32_t)m->n_past;
-    STYX_HIP(hipMemcpyAsync(m->d_tok, &m->h_stage[0], 4, hipMemcpyHostToDevice, m->gpu->stream));
-    STYX_HIP(hipMemcpyAsync(m->d_pos, &m->h_stage[1], 4, hipMemcpyHostToDevice, m->gpu->stream));
+    STYX_HIP(launch_set_token(m->gpu->stream, m->d_tok, m->d_pos, token, m->n_past));
     if (int r = m->run_token(false)) return r;
     m->n_past++;
     if (logits_out)
         STYX_HIP(hipMemcpyAsync(logits_out, m->logits, sizeof(float) * m->V, hipMemcpyDeviceToHost,
                                 m->gpu->stream));
-    m->queue_abort_read();
     STYX_HIP(hipStreamSynchronize(m->gpu->stream));
     if (m->check_abort()) {
-        // the token again (same token and position, still in the stage), on
-        // the separate kernels
+        // the token again (same token and position), on the separate kernels
         if (int r = m->fall_back_unfused()) return r;
         if (int r = m->collect_stats()) return r;
         m->n_past--;
-        STYX_HIP(hipMemcpyAsync(m->d_tok, &m->h_stage[0], 4, hipMemcpyHostToDevice, m->gpu->stream));
-        STYX_HIP(hipMemcpyAsync(m->d_pos, &m->h_stage[1], 4, hipMemcpyHostToDevice, m->gpu->stream));
+        STYX_HIP(launch_set_token(m->gpu->stream, m->d_tok, m->d_pos, token, m->n_past));
         if (int r = m->run_token(false)) return r;
         m->n_past++;
         if (logits_out)
@@ -2095,12 +2094,9 @@ int styx_moe_decode(styx_moe *m, int n_steps, uint32_t *out)
     STYX_HIP(hipSetDevice(m->gpu->device));
     const int start = m->n_past;  // position of the pending (argmax) token
     if (int r = m->ensure_pages(start + n_steps - 1)) return r;
-    m->h_stage[1] = (uint32_t)start;
-    STYX_HIP(hipMemcpyAsync(m->d_pos, &m->h_stage[1], 4, hipMemcpyHostToDevice, m->gpu->stream));
-    // the pending token, for a run again after a fused launch gives up
-    // (every step's argmax overwrites it)
-    if (!m->opts.no_fuse)
-        STYX_HIP(hipMemcpyAsync(m->tok_save, m->d_tok, 4, hipMemcpyDeviceToDevice, m->gpu->stream));
+    // the position, and the pending token kept for a run again after a fused
+    // launch gives up (every step's argmax overwrites it)
+    STYX_HIP(launch_set_token(m->gpu->stream, m->d_tok, m->d_pos, 0, start, true, m->tok_save));
     const bool host_work = (m->opts.repin_interval > 0 && m->any_host) || m->opts.time_kernels;
     // With host work between tokens every step is waited for anyway, so a
     // fused launch that gives up is caught at its own step: the steps before
@@ -2121,14 +2117,11 @@ int styx_moe_decode(styx_moe *m, int n_steps, uint32_t *out)
         if (int r = m->run_token(true)) return r;
         m->n_past++;
         if (host_work && !m->opts.no_fuse) {
-            m->queue_abort_read();
             STYX_HIP(hipStreamSynchronize(m->gpu->stream));
             if (m->check_abort()) {
                 if (int r = m->fall_back_unfused()) return r;
                 m->n_past--;
-                m->h_stage[1] = (uint32_t)m->n_past;
-                STYX_HIP(hipMemcpyAsync(m->d_pos, &m->h_stage[1], 4, hipMemcpyHostToDevice,
-                                        m->gpu->stream));
+                STYX_HIP(launch_set_token(m->gpu->stream, m->d_tok, m->d_pos, 0, m->n_past, true));
                 // the step's input token: the pending one, or the previous step's
                 STYX_HIP(hipMemcpyAsync(m->d_tok, i == 0 ? m->tok_save : m->hist + start + i, 4,
                                         hipMemcpyDeviceToDevice, m->gpu->stream));
@@ -2139,7 +2132,6 @@ int styx_moe_decode(styx_moe *m, int n_steps, uint32_t *out)
     }
     STYX_HIP(hipMemcpyAsync(out, m->hist + start + 1, sizeof(uint32_t) * n_steps,
                             hipMemcpyDeviceToHost, m->gpu->stream));
-    m->queue_abort_read();
     STYX_HIP(hipStreamSynchronize(m->gpu->stream));
     if (m->check_abort()) {
         // the steps again from the pending token, on the separate kernels
@@ -2182,8 +2174,9 @@ int styx_moe_generate(styx_moe *m, const uint32_t *prompt, int n_prompt, int n_p
     for (; i < n_prompt; i++)
         if (int r = styx_moe_forward_token(m, prompt[i], nullptr)) return r;
     const auto t1 = clk::now();
-    // the first generated token is the prefill's argmax, already on device
-    STYX_HIP(hipMemcpy(out, m->d_tok, 4, hipMemcpyDeviceToHost));
+    // the first generated token is the prefill's argmax, left in the stage by
+    // its read-out
+    out[0] = m->h_stage[5];
     if (int r = styx_moe_decode(m, n_predict - 1, out + 1)) return r;
     const auto t2 = clk::now();
     if (prefill_s) *prefill_s = std::chrono::duration<double>(t1 - t0).count();

@@ -275,9 +275,15 @@ hipError_t launch_argmax(hipStream_t st, const float *v, int n, uint32_t *out_to
                          uint32_t *hist);
 // The token of a running argmax word that launch_dense(..., amax) filled
 // (argmax_key order): written to out_tok (and hist[pos+1], pos advanced when
-// advance != 0); the word is cleared for the next launch.
+// advance != 0); the word is cleared for the next launch.  host (optional,
+// mapped host memory) gets {*abort, token}.
 hipError_t launch_argmax_word(hipStream_t st, unsigned long long *amax, uint32_t *out_tok,
-                              int32_t *pos, int advance, uint32_t *hist);
+                              int32_t *pos, int advance, uint32_t *hist, const int *abort = nullptr,
+                              uint2 *host = nullptr);
+// *pos = position, and *tok = token; or, with keep, *tok stays and goes to
+// *saved (optional).
+hipError_t launch_set_token(hipStream_t st, uint32_t *tok, int32_t *pos, uint32_t token,
+                            int32_t position, bool keep = false, uint32_t *saved = nullptr);
 
 // gather_slabs_f32 semantics: for slot s<k with arena id != SKIP copy expert
 // ids[s]'s slab of each tensor into arena slot ids[32+s].

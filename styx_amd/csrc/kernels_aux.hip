@@ -320,13 +320,19 @@ __global__ void __launch_bounds__(64) k_argmax_final(const float *part_key,
     }
 }
 
+// The token's read-out also leaves {abort flag, token} in pinned host memory
+// (host): the caller finds both there after its synchronisation, where copies
+// queued behind the token cost it a blit kernel each.
 __global__ void __launch_bounds__(64) k_argmax_word(unsigned long long *amax, uint32_t *out_tok,
-                                                    int32_t *pos, int advance, uint32_t *hist)
+                                                    int32_t *pos, int advance, uint32_t *hist,
+                                                    const int *abort, uint2 *host)
 {
     if (threadIdx.x != 0) return;
-    // both loads before any store (one memory round trip, not two)
+    // every load before any store (one memory round trip, not two)
     const uint32_t idx = (uint32_t)*amax;
     const int32_t p = advance ? *pos + 1 : 0;
+    const uint32_t ab = host ? (uint32_t)*abort : 0;
+    if (host) *host = make_uint2(ab, idx);
     *amax = 0ull;
     *out_tok = idx;
     if (advance) {
@@ -336,10 +342,32 @@ __global__ void __launch_bounds__(64) k_argmax_word(unsigned long long *amax, ui
 }
 
 hipError_t launch_argmax_word(hipStream_t st, unsigned long long *amax, uint32_t *out_tok,
-                              int32_t *pos, int advance, uint32_t *hist)
+                              int32_t *pos, int advance, uint32_t *hist, const int *abort,
+                              uint2 *host)
 {
-    if (!amax || !out_tok || (advance && !pos)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_argmax_word, dim3(1), dim3(64), 0, st, amax, out_tok, pos, advance, hist);
+    if (!amax || !out_tok || (advance && !pos) || (host && !abort)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_argmax_word, dim3(1), dim3(64), 0, st, amax, out_tok, pos, advance, hist,
+                       abort, host);
+    return hipGetLastError();
+}
+
+// A token's inputs by value: *tok = token unless keep (then *saved = *tok if
+// saved), *pos = position.  One launch in place of a copy per word.
+__global__ void __launch_bounds__(64) k_set_token(uint32_t *tok, int32_t *pos, uint32_t token,
+                                                  int32_t position, int keep, uint32_t *saved)
+{
+    if (threadIdx.x != 0) return;
+    if (!keep)
+        *tok = token;
+    else if (saved)
+        *saved = *tok;
+    *pos = position;
+}
+
+hipError_t launch_set_token(hipStream_t st, uint32_t *tok, int32_t *pos, uint32_t token,
+                            int32_t position, bool keep, uint32_t *saved)
+{
+    hipLaunchKernelGGL(k_set_token, dim3(1), dim3(64), 0, st, tok, pos, token, position, keep ? 1 : 0, saved);
     return hipGetLastError();
 }
 

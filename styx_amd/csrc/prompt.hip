@@ -550,7 +550,7 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
 // k / E = 8 / 128 and two workgroups on a CU.  At 383 tokens of the 30B-A3B
 // shape: q/k/v (5120 x 2048 q8_0) 48 us, gate (q4_K) 87, up (q5_K) 111, down
 // (q6_K) 90 us for 417 MB of slabs; a 384-token prompt through two such
-// layers took 51.7 ms token by token and takes 1.05 ms (with two generated
+// layers took 51.7 ms token by token and takes 1.0 ms (with two generated
 // tokens), the batch itself 0.53 ms.
 template <int T, bool D8, int TT, int NG, int NW>
 __global__ void __launch_bounds__(64 * NW, 2) k_prompt_gemm(PromptGemm a)
