@@ -331,8 +331,8 @@ constexpr int PROMPT_MAX_N = 15360;  // longest activation row (60 KiB of LDS)
 
 // Activation rows as three f16 pieces of x 2^e, [3][rows][np] (np: n rounded
 // up to whole 256-value steps, zeros past n), the sums of each run of 32
-// values as pieces of sum 2^(e-6), [rows][np/256][4][8] (the fourth piece
-// zero), and 2^-e per row.
+// values as pieces of sum 2^(e-6), [rows][np/256][4][8] (third, second, first
+// piece, zeros), and 2^-e per row.
 struct PromptVec {
     uint16_t *p, *sums;
     float *scale;

@@ -16,20 +16,23 @@
 //   k_prompt_router, k_prompt_topk, k_prompt_plan
 //                    router logits, top-k, tokens grouped by expert
 //
-// Precision.  Nothing is held in fewer bits than in the single-token path.
-// Quant values times their 6-bit (q4_K, q5_K) sub-block scale are integers
-// below 2048, q8_0 and q6_K quants are integers below 128: all exact in f16
-// (q6_K's 12-bit products with its 8-bit scale are an f16 plus an exact
-// remainder).  An activation row is scaled by a power of two so that its
-// largest value lies in [2^13, 2^14) and written as three f16 pieces
-// x = p1 + p2 + p3, each the rounding of what the previous ones leave: 33
-// bits below the row's maximum.  v_mfma_f32_16x16x32_f16 forms exact products
-// and f32 sums; a matrix's f16 block factor multiplies the block's sum in
-// f32.  The products of p2 and p3 are summed apart from those of p1 and
-// added in f32: given as the accumulator input of the p1 product, their low
-// bits were dropped downwards by the matrix core, an error of one sign
-// (-0.3 ulp on average over q8_0 rows) that attention over many keys does
-// not average out.
+// Precision.  A row of K/V left here is as close to 64-bit arithmetic as the
+// single-token path's.  Quant values times their 6-bit (q4_K, q5_K) sub-block
+// scale are integers below 2048, q8_0 and q6_K quants are integers below 128:
+// all exact in f16 (q6_K's 12-bit products with its 8-bit scale are an f16
+// plus an exact remainder).  An activation row is scaled by a power of two so
+// that its largest value lies in [2^13, 2^14) and written as three f16 pieces
+// x = p1 + p2 + p3, p1 a multiple of 16 and p2 of 2^-7: 33 bits below the
+// row's maximum.  v_mfma_f32_16x16x32_f16 forms exact products, and sums of
+// integers below 2^24 are exact in its f32 accumulator, so p1's products of
+// 256 values (integers times 16) are summed without an error to speak of; the
+// products of p2 and p3 go into an accumulator of their own.  (With pieces
+// that are each the rounding of what the previous ones leave, the low bits of
+// every addition were dropped downwards by the matrix core.)  A matrix's f16
+// block factor multiplies the block's sum, and blocks are added up, in f64.
+// Layer-0 V rows against 64 bits, relative L2, here and token by token: q8_0
+// 7.1e-8, 8.6e-8; q4_K 9.8e-8, 1.02e-7; q5_K 9.8e-8, 1.06e-7; q6_K 5.9e-8,
+// 9.0e-8 (2048 columns, 300 tokens).
 #include "attn16.h"
 #include "deq.h"
 #include "head.h"
@@ -43,6 +46,7 @@ namespace styx {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef double d4 __attribute__((ext_vector_type(4)));
 
 constexpr int PWG = 256;                 // threads of every kernel here but the plan
 constexpr int KC = 256;                  // values of a row per GEMM step
@@ -76,7 +80,8 @@ hipError_t launch_prompt_embed(hipStream_t st, int t, const uint8_t *w, int64_t 
 //                 moe_reduce_f32.comp:8-13), += sigmoid(gate) y_sh
 //                 (axpy_sig_f32.comp), written back; then as PACK_NORM
 // and the pieces of v, the sums of its runs of 32 (the minimum terms of
-// q4_K / q5_K) as pieces scaled by a further 2^-6, and 2^-e of the row.
+// q4_K / q5_K; formed in f64) as pieces scaled by a further 2^-6, the third
+// piece first, and 2^-e of the row.
 __device__ __forceinline__ float pack_max(float v, float *red)
 {
     v = wave_max(v);
@@ -86,12 +91,23 @@ __device__ __forceinline__ float pack_max(float v, float *red)
     return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-__device__ __forceinline__ void pieces3(float v, _Float16 &a, _Float16 &b, _Float16 &c)
+// v = a + b + c: a a multiple of 16, b of 2^-7, c the rest (|v| < 2^14)
+template <typename F> __device__ __forceinline__ void pieces3(F v, _Float16 &a, _Float16 &b, _Float16 &c)
 {
-    a = (_Float16)v;
-    const float r1 = v - (float)a;
-    b = (_Float16)r1;
-    c = (_Float16)(r1 - (float)b);
+    // adding and taking off 1.5 2^p u, p the mantissa's length, rounds to a
+    // multiple of u
+    constexpr F mid = sizeof(F) == 4 ? (F)12582912.0 : (F)6755399441055744.0;
+    constexpr F g1 = mid * (F)16, g2 = mid * (F)0.0078125;
+    const F p1 = (v + g1) - g1, r1 = v - p1, p2 = (r1 + g2) - g2;
+    a = (_Float16)(float)p1;
+    b = (_Float16)(float)p2;
+    c = (_Float16)(float)(r1 - p2);
+}
+// v of the lane that the DPP control CTRL names
+template <int CTRL> __device__ __forceinline__ double dpp_d(double v)
+{
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    return __longlong_as_double((long long)join64(dpp_u<CTRL>((uint32_t)(u >> 32)), dpp_u<CTRL>((uint32_t)u)));
 }
 
 template <int MODE> __global__ void __launch_bounds__(PWG) k_prompt_pack(PromptPack a)
@@ -181,7 +197,8 @@ template <int MODE> __global__ void __launch_bounds__(PWG) k_prompt_pack(PromptP
     const int np = a.v.np;
     _Float16 *p1 = (_Float16 *)a.v.p + row * np, *p2 = p1 + a.v.rows * np, *p3 = p2 + a.v.rows * np;
     for (int g = threadIdx.x; g < np / 8; g += PWG) {
-        float v[8], s8 = 0.0f;
+        float v[8];
+        double s8 = 0.0;
         h8 c1, c2, c3;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
@@ -197,16 +214,16 @@ template <int MODE> __global__ void __launch_bounds__(PWG) k_prompt_pack(PromptP
         *(h8 *)(p2 + 8 * g) = c2;
         *(h8 *)(p3 + 8 * g) = c3;
         // the run of 32 is held by four neighbouring lanes
-        s8 += dpp_f<0xB1>(s8);
-        s8 += dpp_f<0x4E>(s8);
+        s8 += dpp_d<0xB1>(s8);
+        s8 += dpp_d<0x4E>(s8);
         if ((g & 3) == 0) {
             _Float16 x, y, z;
-            pieces3(s8 * up * 0.015625f, x, y, z);
+            pieces3(s8 * (double)up * 0.015625, x, y, z);
             const int sb = g >> 2;
             _Float16 *s = (_Float16 *)a.v.sums + (row * (np / KC) + (sb >> 3)) * 32 + (sb & 7);
-            s[0] = x;
+            s[0] = z;
             s[8] = y;
-            s[16] = z;
+            s[16] = x;
             s[24] = (_Float16)0.0f;
         }
     }
@@ -371,11 +388,12 @@ __device__ __forceinline__ void u4v_to(const styx_u4 v, uint32_t *o)
 // acc += the products of a step: xop(t, piece, s) gives the activation
 // operand of token tile t, sop(t) its run sums' (q4_K, q5_K).
 template <int T, bool D8, int NG, int TT, typename XOp, typename SOp>
-__device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp sop, f4 (&acc)[NG][TT])
+__device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp sop, d4 (&acc)[NG][TT])
 {
     const int lane = threadIdx.x & 63, g = lane >> 4;
     auto mm = [](h8 a, h8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); };
     const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto widen = [](f4 v) { return __builtin_convertvector(v, d4); };
     if constexpr (T == T_Q8_0) {
         f4 tot[NG][TT];
 #pragma unroll
@@ -406,18 +424,15 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
                     for (int r = 0; r < NG; r++) {
                         const float d = w[r].factor(2 * i + j);
                         const f4 s = mm(x1, op[r][j], zero) + mm(x2, op[r][j], mm(x3, op[r][j], zero));
-                        tot[r][t] = i + j == 0 ? d * s : tot[r][t] + d * s;
+                        tot[r][t] = (i & 1) + j == 0 ? d * s : tot[r][t] + d * s;
                         // added up here, not kept as products until the end
                         // of the step: left to itself the compiler spills
                         asm volatile("" : "+v"(tot[r][t]));
+                        if ((i & 1) + j == 2) acc[r][t] += widen(tot[r][t]);
                     }
                 }
             }
         }
-#pragma unroll
-        for (int r = 0; r < NG; r++)
-#pragma unroll
-            for (int t = 0; t < TT; t++) acc[r][t] += tot[r][t];
     } else {
         f4 big[NG][TT], small[NG][TT];
 #pragma unroll
@@ -506,7 +521,7 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
                     big[r][t] = mm(x1, op[r], big[r][t]);
                     small[r][t] = mm(x3, op[r], small[r][t]);
                     small[r][t] = mm(x2, op[r], small[r][t]);
-                    if constexpr (T == T_Q6_K) small[r][t] = mm(x1, rem[r], small[r][t]);
+                    if constexpr (T == T_Q6_K) small[r][t] = mm(x1, rem[r], mm(x2, rem[r], small[r][t]));
                 }
             }
             if (s & 1) __builtin_amdgcn_sched_barrier(0);
@@ -514,23 +529,28 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
 #pragma unroll
         for (int r = 0; r < NG; r++) {
             if constexpr (T == T_Q6_K) {
-                const float d = f16f(w[r].d);
+                const double d = f16f(w[r].d);
 #pragma unroll
-                for (int t = 0; t < TT; t++) acc[r][t] += d * (big[r][t] + small[r][t]);
+                for (int t = 0; t < TT; t++) acc[r][t] += d * widen(big[r][t] + small[r][t]);
             } else {
-                // minimum terms: sum_j m_j s_j of the 8 sub-blocks, the three
-                // pieces of s_j in lane groups 0..2 (group 3 multiplies zeros)
+                // minimum terms: sum_j m_j s_j of the 8 sub-blocks, the third
+                // to first pieces of s_j in lane groups 0..2 (group 3
+                // multiplies zeros); the first two and the third summed apart,
+                // each exactly
                 const uint32_t z = w[r].hd.z, hw = w[r].hd.w;
                 h2 e[4];
                 bytes_1024(z & 0x3F3F3F3Fu, e[0], e[1]);
                 bytes_1024(((hw >> 4) & 0x0F0F0F0Fu) | ((z >> 2) & 0x30303030u), e[2], e[3]);
                 const h2 off = dup_h2(-1024.0f);
                 const h8 mv = cat8(e[0] + off, e[1] + off, e[2] + off, e[3] + off);
-                const float d = f16f(w[r].hd.x), dm = -64.0f * f16f(w[r].hd.x >> 16);
+                const h8 mz = {}, mhi = g == 0 ? mz : mv, mlo = g == 0 ? mv : mz;
+                const double d = f16f(w[r].hd.x), dm = -64.0 * f16f(w[r].hd.x >> 16);
 #pragma unroll
                 for (int t = 0; t < TT; t++) {
-                    const f4 mn = mm(sop(t), mv, zero);
-                    acc[r][t] += d * (big[r][t] + small[r][t]) + dm * mn;
+                    const h8 sx = sop(t);
+                    const f4 mn = mm(sx, mhi, zero) + mm(sx, mlo, zero);
+                    acc[r][t] += d * widen(big[r][t] + small[r][t]);
+                    acc[r][t] += dm * widen(mn);
                 }
             }
         }
@@ -553,7 +573,7 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
 // layers took 51.7 ms token by token and takes 1.0 ms (with two generated
 // tokens), the batch itself 0.53 ms.
 template <int T, bool D8, int TT, int NG, int NW>
-__global__ void __launch_bounds__(64 * NW, 2) k_prompt_gemm(PromptGemm a)
+__global__ void __launch_bounds__(64 * NW, NW / 2) k_prompt_gemm(PromptGemm a)
 {
     constexpr int TM = 16 * TT, XT = 2 * NW, XR = TM / XT;  // rows staged per pass, passes
     static_assert(TM % XT == 0, "whole passes");
@@ -627,11 +647,11 @@ __global__ void __launch_bounds__(64 * NW, 2) k_prompt_gemm(PromptGemm a)
         if (T == T_Q4_K || T == T_Q5_K)
             if (tid < TM * 4) sr = sb.b128(so, c * 64);
     };
-    f4 acc[NG][TT];
+    d4 acc[NG][TT];
 #pragma unroll
     for (int r = 0; r < NG; r++)
 #pragma unroll
-        for (int t = 0; t < TT; t++) acc[r][t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < TT; t++) acc[r][t] = d4{0.0, 0.0, 0.0, 0.0};
     xload(0);
     wload(0);
     for (int c = 0; c < nc; c++) {
@@ -672,7 +692,7 @@ __global__ void __launch_bounds__(64 * NW, 2) k_prompt_gemm(PromptGemm a)
                 const int row = r0 + 16 * r + n;
                 if (row >= rows) continue;
                 float *y = a.y[seg] + (int64_t)(start + p) * rows + row;
-                const float v = acc[r][t][i] * sc;
+                const float v = (float)acc[r][t][i] * sc;
                 *y = a.add ? *y + v : v;
             }
         }
@@ -688,7 +708,7 @@ __global__ void __launch_bounds__(64 * NW, 2) k_prompt_gemm(PromptGemm a)
 // activations' L2 traffic (every workgroup reads them all) outweighs it.
 template <int T, bool D8, int TT> __global__ void __launch_bounds__(PWG, 2) k_prompt_gemm_few(PromptGemm a)
 {
-    __shared__ f4 s_acc[4][TT][64];
+    __shared__ d4 s_acc[4][TT][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
     int rt = blockIdx.x, seg = 0;
     while (seg + 1 < a.nseg && rt >= a.rt0[seg + 1]) seg++;
@@ -710,9 +730,9 @@ template <int T, bool D8, int TT> __global__ void __launch_bounds__(PWG, 2) k_pr
         so[t] = row * nc * 64 + 16 * g;
     }
     const uint32_t row = min(rt * 16 + n, rows - 1);
-    f4 acc[1][TT];
+    // (the sums stay in LDS between steps: the step's loads need the registers)
 #pragma unroll
-    for (int t = 0; t < TT; t++) acc[0][t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int t = 0; t < TT; t++) s_acc[wave][t][lane] = d4{0.0, 0.0, 0.0, 0.0};
     for (int c = wave; c < nc; c += 4) {
         // every load of the step before any product: one round trip a step
         PW<T, D8> w[1];
@@ -727,22 +747,25 @@ template <int T, bool D8, int TT> __global__ void __launch_bounds__(PWG, 2) k_pr
             if (T == T_Q4_K || T == T_Q5_K) xs[t] = sb.b128(so[t], c * 64);
         }
         __builtin_amdgcn_sched_barrier(0);
+        d4 acc[1][TT];
+#pragma unroll
+        for (int t = 0; t < TT; t++) acc[0][t] = d4{0.0, 0.0, 0.0, 0.0};
         gemm_step<T, D8, 1, TT>(
             w, [&](int t, int p, int s) { return __builtin_bit_cast(h8, x[t][p][s]); },
             [&](int t) { return __builtin_bit_cast(h8, xs[t]); }, acc);
-    }
 #pragma unroll
-    for (int t = 0; t < TT; t++) s_acc[wave][t][lane] = acc[0][t];
+        for (int t = 0; t < TT; t++) s_acc[wave][t][lane] += acc[0][t];
+    }
     __syncthreads();
     if (wave >= TT) return;
     const int t = wave;
-    const f4 v = (s_acc[0][t][lane] + s_acc[1][t][lane]) + (s_acc[2][t][lane] + s_acc[3][t][lane]);
+    const d4 v = (s_acc[0][t][lane] + s_acc[1][t][lane]) + (s_acc[2][t][lane] + s_acc[3][t][lane]);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int p = 16 * t + 4 * g + i;
         if (p >= a.T || rt * 16 + n >= rows) continue;
         float *y = a.y[seg] + (int64_t)p * rows + rt * 16 + n;
-        const float r = v[i] * a.x.scale[p];
+        const float r = (float)v[i] * a.x.scale[p];
         *y = a.add ? *y + r : r;
     }
 }
@@ -779,17 +802,18 @@ template <int T, bool D8, int TT, int NG, int NW> static hipError_t gemm_go(hipS
 template <int T, bool D8 = true> static hipError_t gemm_t(hipStream_t st, PromptGemm &a)
 {
     // 32 positions a tile unless 16 hold them all; eight waves of 16 rows
-    // unless that would leave CUs without a workgroup, then four.  Four waves
-    // of two row tiles each (half the LDS reads per product, 220 registers)
-    // measured the same but for q5_K, whose unpacking takes the most
-    // registers: 111 against 119 us for the up slabs of 383 tokens.
+    // unless that would leave CUs without a workgroup, then four.  q4_K and
+    // q5_K take four waves of two row tiles each (half the LDS reads per
+    // product): the gate slabs (q4_K) of 383 tokens of the 30B-A3B shape 87
+    // us, 93 with eight waves, whose 128 registers do not hold q5_K's
+    // unpacking at all (24 spilled).  q6_K: 92 that way, 89 with eight.
     const int64_t rows = (int64_t)a.rows[0] + (a.nseg > 1 ? a.rows[1] : 0) + (a.nseg > 2 ? a.rows[2] : 0);
     if (!a.tiles && a.T <= 32) return gemm_few<T, D8>(st, a);
     const int tm = a.tile_tokens;
     const int64_t wg = (rows + 127) / 128 * (a.tiles ? a.max_tiles : (a.T + tm - 1) / tm);
     if (tm == 16) return wg < 256 ? gemm_go<T, D8, 1, 1, 4>(st, a) : gemm_go<T, D8, 1, 1, 8>(st, a);
     if (wg < 256) return gemm_go<T, D8, 2, 1, 4>(st, a);
-    if constexpr (T == T_Q5_K) return gemm_go<T, D8, 2, 2, 4>(st, a);
+    if constexpr (T == T_Q4_K || T == T_Q5_K) return gemm_go<T, D8, 2, 2, 4>(st, a);
     return gemm_go<T, D8, 2, 1, 8>(st, a);
 }
 
@@ -908,16 +932,21 @@ __global__ void __launch_bounds__(PWG) k_prompt_router(const float *xn, const fl
     const float *xp = xn + (int64_t)min(t0 + n, T - 1) * H + wave * q + 4 * g;
     const float *wp = W + (int64_t)min(e0 + n, E - 1) * H + wave * q + 4 * g;
     const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    f4 acc[4] = {zero, zero, zero, zero};
-#pragma unroll 4
-    for (int i = 0; i < q; i += 16) {
-        const f4 x = *(const f4 *)(xp + i), w = *(const f4 *)(wp + i);
+    d4 tot = {0.0, 0.0, 0.0, 0.0};
+    // 64 columns' products summed in f32, those sums in f64
+    for (int i = 0; i < q; i += 64) {
+        f4 acc[4] = {zero, zero, zero, zero};
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[e], acc[e], 0, 0, 0);
+        for (int j = 0; j < 64; j += 16) {
+            const f4 x = *(const f4 *)(xp + i + j), w = *(const f4 *)(wp + i + j);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[e], acc[e], 0, 0, 0);
+        }
+        tot += __builtin_convertvector((acc[0] + acc[1]) + (acc[2] + acc[3]), d4);
     }
-    const f4 s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
 #pragma unroll
-    for (int i = 0; i < 4; i++) part[wave][4 * g + i][n] = s[i];
+    for (int i = 0; i < 4; i++) part[wave][4 * g + i][n] = (float)tot[i];
     __syncthreads();
     const int t = threadIdx.x >> 4, e = threadIdx.x & 15;
     if (t0 + t >= T || e0 + e >= E) return;
@@ -1023,7 +1052,7 @@ hipError_t launch_prompt_stage(hipStream_t st, const int *list, const int *ncold
 
 hipError_t launch_prompt_route(hipStream_t st, const PromptRoute &a)
 {
-    if (a.T < 1 || a.E < a.k || a.E > MAX_EXPERTS || a.k < 1 || a.k > MAX_TOPK || a.H % 64)
+    if (a.T < 1 || a.E < a.k || a.E > MAX_EXPERTS || a.k < 1 || a.k > MAX_TOPK || a.H % 256)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_prompt_router, dim3((a.T + 15) / 16, (a.E + 15) / 16), dim3(PWG), 0, st, a.xn,
                        a.W, a.bias, a.logits, a.T, a.E, a.H);

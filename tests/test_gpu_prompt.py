@@ -4,7 +4,10 @@ leaves and the logits after it are compared with the same tokens forwarded
 one by one (the path the other engine tests hold to the oracle), and the
 logits with the oracle itself.
 
-Tolerance: every value is an f32 sum of at most 2048 products, whose order
+How exact the rows are is a test of its own, against 64-bit arithmetic of the
+same model: no further off than the token-by-token path's.
+
+Tolerance of the other tests: every value is an f32 sum of at most 2048 products, whose order
 differs between the two paths (forward error about sqrt(n) 2^-24 = 2.7e-6 of
 the result's norm for random signs, and the same again through a second
 layer), so 1e-5 relative L2."""
@@ -14,6 +17,7 @@ import numpy as np
 import pytest
 
 from helpers import oracle_from_model, rel_l2
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -63,6 +67,98 @@ def check(gpu, c, n_prompt, oracle=True, n_ctx=None, **opts):
         for pos, t in enumerate([*prompt.tolist(), *toks.tolist()]):
             ol, *_ = orc.forward(pos, int(t))
         assert rel_l2(la, ol) < 1e-4
+    a.close()
+    b.close()
+
+
+def tensors64(m):
+    out = {}
+    for name in m.tensor_names():
+        t, dims, data = m.export_tensor(name)
+        a = data.view(np.float32) if t == 0 else O.dequant(t, data, int(np.prod(dims)))
+        out[name] = a.astype(np.float64).reshape(dims[::-1])
+    return out
+
+
+def kv64(m, toks):
+    """The first two layers' (K, V) rows of toks at positions 0.. in 64 bits,
+    and each token's routing margin (k-th against k+1-th logit)."""
+    hp, W, T = m.hp, tensors64(m), len(toks)
+    nh, nkv, hd, k, half = hp.n_heads, hp.n_kv_heads, hp.head_dim, hp.n_expert_used, hp.head_dim // 2
+    eps = float(np.float32(hp.rms_eps))
+    norm = lambda x, w: x / np.sqrt((x * x).mean(-1, keepdims=True) + eps) * (1 if w is None else w)
+    silu = lambda v: v / (1 + np.exp(-v))
+    ang = np.arange(T)[:, None] * float(np.float32(hp.rope_base)) ** (-2.0 * np.arange(half) / hd)
+    c, s = np.cos(ang)[:, None, :], np.sin(ang)[:, None, :]
+    rope = lambda x: np.concatenate([x[..., :half] * c - x[..., half:] * s,
+                                     x[..., :half] * s + x[..., half:] * c], -1)
+    x = W["token_embd.weight"][toks]
+    rows = []
+    for l in range(2):
+        w = lambda n: W.get(f"blk.{l}.{n}.weight")
+        h = norm(x, w("attn_norm"))
+        q, kk, v = ((h @ w(n).T).reshape(T, -1, hd) for n in ("attn_q", "attn_k", "attn_v"))
+        if w("attn_q_norm") is not None:
+            q = norm(q, w("attn_q_norm"))
+        if w("attn_k_norm") is not None:
+            kk = norm(kk, w("attn_k_norm"))
+        q, kk = rope(q), rope(kk)
+        rows.append((kk.reshape(T, -1), v.reshape(T, -1)))
+        if l == 1:
+            return rows, margin
+        o = np.empty((T, nh, hd))
+        for i in range(nh):
+            sc = q[:, i] @ kk[:, i * nkv // nh].T / np.sqrt(hd)
+            sc[np.triu_indices(T, 1)] = -np.inf
+            p = np.exp(sc - sc.max(1, keepdims=True))
+            o[:, i] = p / p.sum(1, keepdims=True) @ v[:, i * nkv // nh]
+        x = x + o.reshape(T, -1) @ w("attn_output").T
+        h = norm(x, w("ffn_norm"))
+        lg = h @ w("ffn_gate_inp").T
+        order = np.argsort(-lg, axis=1, kind="stable")
+        top = np.take_along_axis(lg, order, 1)
+        margin = top[:, k - 1] - top[:, k]
+        p = np.exp(top[:, :k] - top[:, :1])
+        p /= p.sum(1, keepdims=True)
+        for e in range(hp.n_expert):
+            t, sl = np.nonzero(order[:, :k] == e)
+            g, u = h[t] @ w("ffn_gate_exps")[e].T, h[t] @ w("ffn_up_exps")[e].T
+            x[t] += p[t, sl][:, None] * ((silu(g) * u) @ w("ffn_down_exps")[e].T)
+
+
+BIG = dict(n_embd=1024, n_heads=32, n_kv_heads=4, n_expert=16, n_expert_used=8)
+
+
+# each type's dense products in their few-token, four-wave and eight-wave (or
+# two-row-tile) forms, and each type in each expert role with enough tokens
+# for the latter; 800 and 1312 rows end inside a workgroup's 128; 8192
+# columns are 32 steps of a workgroup
+@pytest.mark.parametrize("kw,n", [
+    *[(dict(attn_type=t), n) for t in (Q8_0, Q4_K, Q5_K, Q6_K) for n in (20, 70)],
+    *[(dict(n_embd=8192, attn_type=t), 60) for t in (Q8_0, Q4_K, Q6_K)],
+    *[(dict(BIG, attn_type=t, exp_type=e, n_ff_exp=f), 261) for t, e, f in (
+        (Q8_0, (Q4_K, Q5_K, Q8_0), 800), (Q4_K, (Q6_K, Q4_K, Q8_0), 800), (Q5_K, (Q8_0, Q8_0, Q8_0), 1312),
+        (Q6_K, (Q5_K, Q6_K, Q4_K), 768), (Q8_0, (Q5_K, Q4_K, Q5_K), 768), (Q8_0, (Q6_K, Q6_K, Q6_K), 768))],
+])
+def test_rows_as_exact_as_token_by_token(gpu, kw, n):
+    """K/V rows against 64 bits: relative L2 at most 1.05 times that of the
+    tokens forwarded one by one (the two differ only in roundings, so their
+    ratio over 1e5 values moves by about 1%), and no bias: the mean error
+    towards larger values within half an f32 rounding (2^-25)."""
+    from styx_amd import MoeModel
+    c = cfg(**kw)
+    toks = np.random.default_rng(n).integers(0, c.n_vocab, n + 1).astype(np.uint32)
+    a, b = MoeModel.synth(gpu, c, n_ctx=n + 8), MoeModel.synth(gpu, c, n_ctx=n + 8)
+    a.generate(toks, 1)
+    for t in toks:
+        b.forward_token(int(t), False)
+    ref, margin = kv64(b, toks[:n])
+    for layer in (0, 1):
+        sel = margin > 1e-4 if layer else slice(None)  # (tokens routed without a doubt)
+        for x, y, r in zip(a.read_kv(layer, 0, n), b.read_kv(layer, 0, n), ref[layer]):
+            x, y, r = (v.reshape(n, -1)[sel].astype(np.float64) for v in (x, y, r))
+            assert rel_l2(x, r) <= 1.05 * rel_l2(y, r), (layer, rel_l2(x, r), rel_l2(y, r))
+            assert abs((np.sign(r) * (x - r)).mean()) <= 2.0 ** -25 * np.abs(r).mean(), layer
     a.close()
     b.close()
 
