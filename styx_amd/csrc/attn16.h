@@ -10,6 +10,8 @@
 // on both sides of each product.
 #pragma once
 
+#include <algorithm>
+
 #include "qdot.h"
 
 namespace styx {
@@ -169,5 +171,22 @@ __device__ __forceinline__ void attn16_merge(const Attn16<HD> &a, Merge16<HD> &s
         }
     }
 }
+
+// Keys per workgroup of a launch of `groups` workgroups (16 query rows of one
+// kv head each, `rows` rows in all) over n_t keys: all of them up to 256 (two
+// blocks per wave: a merge kernel costs more), else a multiple of 128 (one
+// block per wave) that makes at most 512 workgroups, two per CU, whose
+// partials [rows][chunks][hd + 2] fit `floats`.
+inline uint32_t attn_chunk_keys(uint64_t n_t, uint64_t groups, uint64_t rows, uint64_t hd, uint64_t floats)
+{
+    if (n_t <= 256) return (uint32_t)n_t;
+    const uint64_t most = std::min<uint64_t>(512 / std::min<uint64_t>(groups, 512), floats / (rows * (hd + 2)));
+    if (most < 2) return (uint32_t)n_t;
+    return (uint32_t)std::min<uint64_t>(n_t, (n_t + 128 * most - 1) / (128 * most) * 128);
+}
+
+// O[row][hd] from the chunks' partials {m, l, o[hd]}, part [rows][chunks][hd + 2];
+// at most 512 chunks.
+hipError_t launch_attn_merge(hipStream_t st, const float *part, float *O, int rows, int chunks, int hd);
 
 }  // namespace styx

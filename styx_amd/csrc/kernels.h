@@ -410,6 +410,9 @@ struct PromptAttn {
     int page_tokens, T, pos0, nh, nkv, hd;
     float scale;
     float *out;            // [T][nh*hd]
+    float *part;           // partials of split contexts, part_floats of them
+    uint64_t part_floats;
+    int chunk;             // keys per workgroup, filled by the launch
 };
 
 struct PromptRoute {
@@ -432,7 +435,7 @@ hipError_t launch_prompt_embed(hipStream_t st, int t, const uint8_t *w, int64_t 
 hipError_t launch_prompt_pack(hipStream_t st, int mode, const PromptPack &a, int rows);
 hipError_t launch_prompt_gemm(hipStream_t st, int t, PromptGemm a);
 hipError_t launch_prompt_rope(hipStream_t st, const PromptAttn &a);
-hipError_t launch_prompt_attn(hipStream_t st, const PromptAttn &a);
+hipError_t launch_prompt_attn(hipStream_t st, PromptAttn a);
 // The first `slots` cold experts' slabs of one tensor to dst, slab bytes apart.
 hipError_t launch_prompt_stage(hipStream_t st, const int *list, const int *ncold, const uint8_t *src,
                                int64_t slab, uint8_t *dst, int slots);

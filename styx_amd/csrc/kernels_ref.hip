@@ -174,7 +174,7 @@ template <int HD> __global__ void __launch_bounds__(256) kr_attn16(AttnRef a)
     });
 }
 
-// One workgroup per query head: the chunks' factors in LDS, then 512 / hd
+// One workgroup per query row: the chunks' factors in LDS, then 512 / hd
 // thread groups over every (512 / hd)th chunk, one thread per dimension,
 // eight chunks' loads in flight each (32 chunks: one thread per dimension over
 // all of them took 11 us, this 3.9).  Up to 512 chunks.
@@ -204,16 +204,11 @@ __global__ void __launch_bounds__(AM_WG) kr_attn_merge(const float *part, float 
     O[(int64_t)blockIdx.x * hd + d] = o / L;
 }
 
-// Chunks of a context of n_t keys for ny workgroups per chunk and gx heads:
-// one up to 256 keys (two blocks per wave: a merge kernel costs more), else
-// of 128 keys (one block per wave) while the launch has at most 512
-// workgroups, two per CU, and the partials fit the scratch.
-static uint32_t attn_chunk_keys(uint64_t n_t, uint64_t ny, uint64_t gx, uint64_t hd, const RefScratch *s)
+hipError_t launch_attn_merge(hipStream_t st, const float *part, float *O, int rows, int chunks, int hd)
 {
-    if (n_t <= 256 || !s || !s->p) return (uint32_t)n_t;
-    const uint64_t most = std::min<uint64_t>(512 / std::min<uint64_t>(ny, 512), s->floats / (gx * (hd + 2)));
-    if (most < 2) return (uint32_t)n_t;
-    return (uint32_t)std::min<uint64_t>(n_t, (n_t + 128 * most - 1) / (128 * most) * 128);
+    if (!part || rows < 1 || chunks < 1 || chunks > AM_WG || hd < 1 || AM_WG % hd) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kr_attn_merge, dim3(rows), dim3(AM_WG), 0, st, part, O, chunks, hd);
+    return hipGetLastError();
 }
 
 static hipError_t attn_go(hipStream_t st, AttnRef a, uint32_t hd, const RefScratch *s)
@@ -221,7 +216,7 @@ static hipError_t attn_go(hipStream_t st, AttnRef a, uint32_t hd, const RefScrat
     a.tiles = (a.gqa + 15) / 16;
     const uint64_t ny = (uint64_t)((a.nh + a.gqa - 1) / a.gqa) * a.tiles;
     if (ny > 65535) return hipErrorNotSupported;
-    a.chunk = attn_chunk_keys(a.n_t, ny, a.nh, hd, s);
+    a.chunk = attn_chunk_keys(a.n_t, ny, a.nh, hd, s && s->p ? s->floats : 0);
     const uint32_t chunks = (a.n_t + a.chunk - 1) / a.chunk;
     a.part = chunks > 1 ? s->p : nullptr;
     const dim3 grid(chunks, (unsigned)ny);
@@ -231,7 +226,7 @@ static hipError_t attn_go(hipStream_t st, AttnRef a, uint32_t hd, const RefScrat
         hipLaunchKernelGGL(kr_attn16<128>, grid, dim3(256), 0, st, a);
     else
         hipLaunchKernelGGL(kr_attn16<256>, grid, dim3(256), 0, st, a);
-    if (chunks > 1) hipLaunchKernelGGL(kr_attn_merge, dim3(a.nh), dim3(AM_WG), 0, st, a.part, a.O, (int)chunks, (int)hd);
+    if (chunks > 1) return launch_attn_merge(st, a.part, a.O, (int)a.nh, (int)chunks, (int)hd);
     return hipGetLastError();
 }
 
