@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 namespace styx {
 
@@ -277,8 +278,11 @@ __global__ void __launch_bounds__(256) kr_rms_norm(const float *a, const float *
 // high-nibble ones), so that a lane group of cols / 32 lanes reads a row's
 // blocks end to end in 16-byte loads.  A lane keeps its units' activations
 // in registers over the rows its group visits and has the next row's loads
-// in flight over this row's products, which are f32 FMAs of the integer
-// quants; the unit's factors multiply the sums.
+// in flight over this row's products: f32 FMAs of weights dequantized one by
+// one, as the reference's.  (Factors taken out of the sums, d (s sum q x - m
+// sum x), cost a quarter of the instructions and no time, but cancel: q6_K
+// rows times activations around 1 were 5.0e-7 off 64 bits, so 1.3e-7, and an
+// infinite activation gave NaN where its row's sum is infinite.)
 //
 // Bound: the memory round trip at one expert's few rows, the weight stream
 // beyond.  Against one lane per block and byte loads into a dequantized
@@ -311,29 +315,27 @@ __device__ __forceinline__ styx_u4 ld16(const uint8_t *p) { return *(const styx_
 
 template <int N> __device__ __forceinline__ float ubyte(uint32_t v) { return (float)((v >> (8 * N)) & 255u); }
 
-// sum of 16 unsigned bytes times x[0..16)
-__device__ __forceinline__ float dot16(const styx_u4 q, const float *x)
+template <int N> __device__ __forceinline__ float sbyte(uint32_t v) { return (float)(int8_t)(v >> (8 * N)); }
+
+// sum of y(byte) x over 16 bytes (signed if S) and x[0..16), y the byte's weight
+template <bool S = false, typename Y> __device__ __forceinline__ float dot16(const styx_u4 q, const float *x, Y y)
 {
+    auto b = [&](auto n, int i) { return y(S ? sbyte<decltype(n)::value>(q[i]) : ubyte<decltype(n)::value>(q[i])); };
+    using std::integral_constant;
+    const integral_constant<int, 0> n0;
+    const integral_constant<int, 1> n1;
+    const integral_constant<int, 2> n2;
+    const integral_constant<int, 3> n3;
     float s[4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
-        s[i] = fmaf(ubyte<0>(q[i]), x[4 * i], ubyte<1>(q[i]) * x[4 * i + 1]) +
-               fmaf(ubyte<2>(q[i]), x[4 * i + 2], ubyte<3>(q[i]) * x[4 * i + 3]);
-    return (s[0] + s[1]) + (s[2] + s[3]);
-}
-__device__ __forceinline__ float dot16s(const styx_u4 q, const float *x)  // signed bytes
-{
-    float s[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        s[i] = fmaf((float)(int8_t)q[i], x[4 * i], (float)(int8_t)(q[i] >> 8) * x[4 * i + 1]) +
-               fmaf((float)(int8_t)(q[i] >> 16), x[4 * i + 2], (float)((int32_t)q[i] >> 24) * x[4 * i + 3]);
+        s[i] = fmaf(b(n0, i), x[4 * i], b(n1, i) * x[4 * i + 1]) + fmaf(b(n2, i), x[4 * i + 2], b(n3, i) * x[4 * i + 3]);
     return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
-// One unit's activations: two runs of 16 values and their sums.
+// One unit's activations: two runs of 16 values.
 struct MX {
-    float x[32], s0, s1;
+    float x[32];
     __device__ __forceinline__ void load(const float *b, int lo, int hi)
     {
 #pragma unroll
@@ -342,9 +344,6 @@ struct MX {
 #pragma unroll
             for (int j = 0; j < 4; j++) x[4 * i + j] = u[j], x[16 + 4 * i + j] = v[j];
         }
-        s0 = s1 = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; i++) s0 += x[i], s1 += x[16 + i];
     }
 };
 
@@ -364,7 +363,9 @@ template <> struct MU<T_Q8_0> {
     }
     __device__ __forceinline__ float dot(const MX &x, int) const
     {
-        return f16f(d) * (dot16s(q0, x.x) + dot16s(q1, x.x + 16));
+        const float df = f16f(d);
+        auto y = [=](float v) { return df * v; };
+        return dot16<true>(q0, x.x, y) + dot16<true>(q1, x.x + 16, y);
     }
 };
 // q4_K / q5_K: part p = u & 7 reads quant bytes [16 p, +16): run h = p & 1
@@ -395,8 +396,9 @@ template <int T> struct MUK {
         float s0, s1, m0, m1;
         k4_scales(make_uint4(hd.x, hd.y, hd.z, hd.w), 16 * (c & 1), c >> 1, s0, s1, m0, m1);
         const float d = f16f(hd.x), dm = f16f(hd.x >> 16);
-        return ((d * s0) * dot16(lo, x.x) - (dm * m0) * x.s0) +
-               ((d * s1) * dot16(hi, x.x + 16) - (dm * m1) * x.s1);
+        s0 *= d, s1 *= d, m0 *= dm, m1 *= dm;
+        return dot16(lo, x.x, [=](float u) { return fmaf(s0, u, -m0); }) +
+               dot16(hi, x.x + 16, [=](float u) { return fmaf(s1, u, -m1); });
     }
 };
 template <> struct MU<T_Q4_K> : MUK<T_Q4_K> {};
@@ -427,8 +429,10 @@ template <> struct MU<T_Q6_K> {
         const uint32_t j2 = 2 * ((u >> 1) & 1);
         const styx_u4 lo = (q & 0x0F0F0F0Fu) | (((qh >> j2) & 0x03030303u) << 4);
         const styx_u4 hi = ((q >> 4) & 0x0F0F0F0Fu) | (((qh >> (j2 + 4u)) & 0x03030303u) << 4);
-        const float s0 = (float)(int8_t)sc, s1 = (float)(int8_t)(sc >> 16);
-        return f16f(d) * (s0 * (dot16(lo, x.x) - 32.0f * x.s0) + s1 * (dot16(hi, x.x + 16) - 32.0f * x.s1));
+        const float s0 = f16f(d) * (float)(int8_t)sc, s1 = f16f(d) * (float)(int8_t)(sc >> 16);
+        // s (u - 32) in one rounding: s u and 32 s are exact
+        return dot16(lo, x.x, [=](float u) { return fmaf(s0, u, -32.0f * s0); }) +
+               dot16(hi, x.x + 16, [=](float u) { return fmaf(s1, u, -32.0f * s1); });
     }
 };
 

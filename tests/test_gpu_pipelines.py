@@ -54,6 +54,80 @@ def test_matvec_rows(gpu, t, rows, cols):
     assert (got[rows:] == 9.0).all()
 
 
+def matvec(gpu, t, a, rows, cols, x):
+    be, _ = BLK[t]
+    bd = gpu.zeros(rows * 4)
+    push = struct.pack("<13I", cols, cols // be, cols, rows, rows * cols, cols, rows, 0, 0, 1, 1, 1, 1)
+    run(gpu, f"mul_mat_vec_{NAME[t]}_f32_f32", [gpu.from_numpy(a), f32buf(gpu, x), bd, gpu.zeros(16),
+                                               gpu.zeros(16)], push, (rows, 1, 1), [(1, 1)])
+    return bd.download(np.float32)
+
+
+@pytest.mark.parametrize("t", [8, 12, 13, 14])
+@pytest.mark.parametrize("cols", [256, 2048, 8192])
+def test_matvec_of_activations_around_one(gpu, t, cols):
+    """Nothing cancels but what the weights themselves cancel: a lane adds
+    its values in a tree of 4 levels, its units in turn, the lanes in 6
+    levels, about 16 roundings of random sign in a row: sqrt(16) 2^-24 of the
+    result's norm at most.  (With 32 taken off q6_K's sums instead of its
+    values the error was 5e-7.)"""
+    rows = 512
+    a = weights(t, rows, cols, cols + t)
+    x = (1 + 0.1 * np.random.default_rng(t).standard_normal(cols)).astype(np.float32)
+    assert rel_l2(matvec(gpu, t, a, rows, cols, x), O.matvec_f64(t, a, rows, cols, x)) < 4 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("t", [8, 12, 13, 14])
+@pytest.mark.parametrize("big", [np.inf, -np.inf, 3e38])
+def test_matvec_of_an_infinite_or_huge_activation(gpu, t, big):
+    """As the products of the dequantized weights: an infinity where the
+    weight is not zero, NaN where it is; a value that fits f32 where the
+    product does."""
+    rows, cols = 512, 768
+    a = weights(t, rows, cols, 5 + t)
+    x = np.random.default_rng(3).standard_normal(cols).astype(np.float32)
+    x[77] = big
+    got = matvec(gpu, t, a, rows, cols, x)
+    w = O.dequant(t, a, rows * cols).reshape(rows, cols)[:, 77].astype(np.float64)
+    if np.isinf(big):
+        assert (np.isnan(got) == (w == 0)).all()
+        assert (got[w != 0] == np.sign(w[w != 0]) * big).all()
+    else:
+        y, top = w * float(np.float32(big)), float(np.finfo(np.float32).max)
+        fits, over = np.abs(y) < 0.999 * top, np.abs(y) > 1.001 * top
+        assert fits.any() and over.any() and np.isfinite(got[fits]).all()
+        assert (got[over] == np.sign(y[over]) * np.inf).all()
+        assert (np.abs(got[fits] - y[fits]) <= 1e-6 * np.abs(y[fits]) + 1e30).all()
+
+
+# two passes of rows per lane group and a ragged last one: one, two and more
+# units per lane
+@pytest.mark.parametrize("t,rows,cols", [(8, 4099, 2048), (12, 4100, 4096), (13, 4104, 4608), (14, 4101, 4608),
+                                         (14, 4099, 2048), (12, 8209, 1024)])
+def test_matvec_several_passes(gpu, t, rows, cols):
+    test_matvec_rows(gpu, t, rows, cols)
+
+
+def test_matvec_id_several_passes(gpu):
+    """8 slots x 2049 rows of 16 lanes: two passes, the last of one row."""
+    t, E, rows, cols, k = 14, 3, 2049, 512, 8
+    be, bb = BLK[t]
+    a = weights(t, E * rows, cols, 21)
+    x = np.random.default_rng(4).standard_normal(cols).astype(np.float32)
+    ids = np.array([2, 0, 1, 1, 0, 2, 2, 1], np.int32)
+    bd = f32buf(gpu, np.full(k * rows + 5, 9.0))
+    run(gpu, f"mul_mat_vec_id_{NAME[t]}_f32_f32",
+        [gpu.from_numpy(a), f32buf(gpu, x), bd, gpu.zeros(16), gpu.zeros(16), gpu.from_numpy(ids)],
+        mmv_id_push(cols, rows, be, k), (rows, k, 1))
+    got = bd.download(np.float32)
+    n = rows * (cols // be) * bb
+    for s, e in enumerate(ids):
+        w = a[e * n:(e + 1) * n]
+        assert (np.abs(got[s * rows:(s + 1) * rows] - O.matvec_f64(t, w, rows, cols, x))
+                <= sum_bound(t, w, rows, cols, x)).all()
+    assert (got[k * rows:] == 9.0).all()
+
+
 def test_matvec_grid_covers_part_of_the_rows(gpu):
     """NUM_ROWS rows per workgroup of the reference grid, and no row past it."""
     t, rows, cols = 12, 64, 512
