@@ -64,7 +64,9 @@ template <int HD> struct Attn16 {
 
     // A block of keys: rows `stride` floats apart at kb / vb, of which rows
     // past lim are not read and those at or past vis are not seen by this
-    // lane's query.
+    // lane's query.  Those meet a factor 0 (rows past lim: times row lim
+    // again), which a V value that is not finite turns into NaN: the callers
+    // see to that.
     __device__ __forceinline__ void block(const float *kb, const float *vb, int64_t stride, int lim,
                                           int vis, float scale)
     {

@@ -165,6 +165,18 @@ template <int HD> __global__ void __launch_bounds__(256) kr_attn16(AttnRef a)
     attn16_merge<HD>(at, s, [&](int r, int d, float O, float L, float M) {
         if ((uint32_t)r >= nrow) return;
         const int64_t h = h0 + r;
+        // the last block's missing keys are 0 times its last row: where that
+        // holds an infinity, the keys' own sum
+        if (O != O && isinf(a.V[(int64_t)(c1 - 1) * a.kv_dim + (int64_t)kvh * HD + d])) {
+            O = 0.0f;
+            for (uint32_t k = c0; k < c1; k++) {
+                const int64_t row = (int64_t)k * a.kv_dim + (int64_t)kvh * HD;
+                float x = 0.0f;
+#pragma unroll 4
+                for (int i = 0; i < HD; i++) x += a.Q[h * HD + i] * a.K[row + i];
+                O += expf(x * a.scale - M) * a.V[row + d];
+            }
+        }
         if (!a.part) {
             a.O[h * HD + d] = O / L;
             return;

@@ -201,6 +201,27 @@ def test_attn_decode_shapes(gpu, n_t, hd, nh, gqa, pad):
     assert (got[nh * hd:] == 3.0).all()
 
 
+# contexts that end inside a key block, one and several chunks
+@pytest.mark.parametrize("n_t,hd,gqa", [(1, 64, 1), (31, 128, 4), (32, 128, 4), (33, 256, 2), (257, 64, 8),
+                                        (600, 128, 4)])
+@pytest.mark.parametrize("at", [0, -1])
+def test_attn_decode_infinite_value(gpu, n_t, hd, gqa, at):
+    """An infinity in the first or last V row: an infinity in that dimension
+    of the heads that read it, every other output as without."""
+    rng = np.random.default_rng(n_t)
+    nh, kvd, scale = 2 * gqa, 2 * hd, np.float32(1 / np.sqrt(hd))
+    q, K, V = (rng.standard_normal(n).astype(np.float32) for n in (nh * hd, n_t * kvd, n_t * kvd))
+    ref = O.attn_decode_f64(q, K, V, n_t, hd, kvd, gqa, nh, float(scale)).reshape(nh, hd)
+    V.reshape(n_t, kvd)[at, 3] = -np.inf
+    bo = gpu.zeros(nh * hd * 4)
+    run(gpu, "attn_decode_f32", [f32buf(gpu, q), f32buf(gpu, K), f32buf(gpu, V), bo],
+        struct.pack("<4If", n_t, hd, kvd, gqa, scale), (nh, 1, 1))
+    got = bo.download(np.float32).reshape(nh, hd)
+    assert (got[:gqa, 3] == -np.inf).all()
+    got[:gqa, 3] = ref[:gqa, 3] = 0
+    assert rel_l2(got, ref) < 2e-6
+
+
 def test_attn_in_async_and_plain_batches(gpu):
     """Split contexts on two streams at once: each batch has its own partials."""
     from styx_amd.runtime import Batch, Kernel, Timeline
