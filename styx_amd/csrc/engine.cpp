@@ -195,7 +195,7 @@ struct styx_moe {
         float *x, *xn, *q, *k, *v, *attn, *part, *logits, *wts, *g, *u, *y, *sh_y, *gate;
         int32_t *ids, *order, *inv;
         int4 *tiles;
-        int *ntiles;
+        int *ntiles, *odd;
         void *vec_h, *vec_o, *vec_f;  // pieces of H-, q_dim- and F-wide rows
         // experts in host memory: the cold ones of a layer, and a buffer that
         // one of its tensors' cold slabs pass through (those that fit)
@@ -1053,6 +1053,7 @@ int styx_moe::prompt_workspace()
         put(&w.inv, 4 * P);
         put(&w.tiles, sizeof(int4) * (P / 16 + E));
         put(&w.ntiles, 4);
+        put(&w.odd, 4);
         put((char **)&w.vec_h, prompt_vec_bytes(T, H));
         put((char **)&w.vec_o, prompt_vec_bytes(T, (int)qd));
         put(&w.cold_slot, 4 * (size_t)E);
@@ -1075,7 +1076,7 @@ int styx_moe::prompt_workspace()
     };
     at(&pb.tok), at(&pb.x), at(&pb.xn), at(&pb.q), at(&pb.k), at(&pb.v), at(&pb.attn), at(&pb.part);
     at(&pb.logits), at(&pb.wts), at(&pb.g), at(&pb.u), at(&pb.y), at(&pb.sh_y), at(&pb.gate);
-    at(&pb.ids), at(&pb.order), at(&pb.inv), at(&pb.tiles), at(&pb.ntiles);
+    at(&pb.ids), at(&pb.order), at(&pb.inv), at(&pb.tiles), at(&pb.ntiles), at(&pb.odd);
     at((char **)&pb.vec_h), at((char **)&pb.vec_o), at((char **)&pb.vec_f);
     at(&pb.cold_slot), at(&pb.cold_list), at(&pb.ncold), at(&pb.stage);
     pb_t = T;
@@ -1098,7 +1099,7 @@ int styx_moe::prompt_batch(const uint32_t *tok, int n)
         // meets on average with some room above it
         const int td = T <= 16 ? 16 : 32, te = P <= 12 * E ? 16 : 32;
         CK(hipMemcpyAsync(pb.tok, tok, 4 * (size_t)T, hipMemcpyHostToDevice, st));
-        CK(launch_prompt_embed(st, embd.type, embd.dev, V, H, pb.tok, T, pb.x));
+        CK(launch_prompt_embed(st, embd.type, embd.dev, V, H, pb.tok, T, pb.x, pb.odd));
         auto pack = [&](int mode, float *src, const PromptVec &v, int rows, auto fill) {
             PromptPack p{};
             p.src = src;
@@ -1155,6 +1156,7 @@ int styx_moe::prompt_batch(const uint32_t *tok, int n)
             a.hd = hd;
             a.scale = 1.0f / std::sqrt((float)hd);
             a.out = pb.attn;
+            a.odd = pb.odd;
             a.part = pb.part;
             a.part_floats = pb_part();
             CK(launch_prompt_rope(st, a));

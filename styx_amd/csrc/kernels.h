@@ -413,6 +413,7 @@ struct PromptAttn {
     float *part;           // partials of split contexts, part_floats of them
     uint64_t part_floats;
     int chunk;             // keys per workgroup, filled by the launch
+    int *odd;              // whether the batch wrote a V value that is not finite
 };
 
 struct PromptRoute {
@@ -431,7 +432,7 @@ struct PromptRoute {
 };
 
 hipError_t launch_prompt_embed(hipStream_t st, int t, const uint8_t *w, int64_t nrows, int ncols,
-                               const uint32_t *tok, int T, float *x);
+                               const uint32_t *tok, int T, float *x, int *odd);
 hipError_t launch_prompt_pack(hipStream_t st, int mode, const PromptPack &a, int rows);
 hipError_t launch_prompt_gemm(hipStream_t st, int t, PromptGemm a);
 hipError_t launch_prompt_rope(hipStream_t st, const PromptAttn &a);

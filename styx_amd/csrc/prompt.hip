@@ -7,7 +7,7 @@
 // together, so that each matrix and each routed expert's slab is read once
 // per 32 tokens that use it, and the contraction runs on the matrix cores:
 //
-//   k_prompt_embed   residual rows of the tokens
+//   k_prompt_embed   residual rows of the tokens; clears the batch's odd flag
 //   k_prompt_pack    a row's RMSNorm / SwiGLU / combine, and its f16 pieces
 //   k_prompt_gemm    split-layout quant matrix x token rows (dense matrices,
 //                    or the tokens of each routed expert)
@@ -54,8 +54,10 @@ constexpr int XROW = KC * 2 + 16;        // bytes of a token's piece of a step i
 
 // ------------------------------------------------------------ embedding ----
 __global__ void __launch_bounds__(PWG) k_prompt_embed(int t, const uint8_t *w, int64_t nrows,
-                                                      int ncols, const uint32_t *tok, float *x)
+                                                      int ncols, const uint32_t *tok, float *x,
+                                                      int *odd)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *odd = 0;
     const int be = blk_elems(t), nb = ncols / be;
     const Mat m = mat_at(w, t, nrows * nb);
     const int64_t r = tok[blockIdx.x];
@@ -64,10 +66,10 @@ __global__ void __launch_bounds__(PWG) k_prompt_embed(int t, const uint8_t *w, i
 }
 
 hipError_t launch_prompt_embed(hipStream_t st, int t, const uint8_t *w, int64_t nrows, int ncols,
-                               const uint32_t *tok, int T, float *x)
+                               const uint32_t *tok, int T, float *x, int *odd)
 {
-    if (T < 1 || ncols % blk_elems(t)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_prompt_embed, dim3(T), dim3(PWG), 0, st, t, w, nrows, ncols, tok, x);
+    if (T < 1 || !odd || ncols % blk_elems(t)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_prompt_embed, dim3(T), dim3(PWG), 0, st, t, w, nrows, ncols, tok, x, odd);
     return hipGetLastError();
 }
 
@@ -839,7 +841,8 @@ hipError_t launch_prompt_gemm(hipStream_t st, int t, PromptGemm a)
 
 // ------------------------------------------------------- rope, K/V rows ----
 // One workgroup per token: its q heads normalised and rotated in place, its
-// k heads into the K cache, its v heads into the V cache.
+// k heads into the K cache, its v heads into the V cache; *odd set if one of
+// their values is not finite.
 template <int PPL> __global__ void __launch_bounds__(PWG) k_prompt_rope(PromptAttn a)
 {
     const int t = blockIdx.x, pos = a.pos0 + t, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -859,7 +862,11 @@ template <int PPL> __global__ void __launch_bounds__(PWG) k_prompt_rope(PromptAt
         HeadIn<PPL> in;
         head_load<PPL>(in, a.k + o, a.k_norm, a.hd);
         head_finish<PPL>(in, cs, a.k_norm != nullptr, a.eps, a.hd, a.kpool + at(h));
-        for (int i = lane; i < a.hd; i += 64) a.vpool[at(h) + i] = a.v[o + i];
+        for (int i = lane; i < a.hd; i += 64) {
+            const float v = a.v[o + i];
+            a.vpool[at(h) + i] = v;
+            if (!(fabsf(v) < INFINITY)) *a.odd = 1;
+        }
     }
 }
 
@@ -873,9 +880,69 @@ template <int PPL> __global__ void __launch_bounds__(PWG) k_prompt_rope(PromptAt
 // quarter of the keys in turn.  A prompt of five tokens after 32000 keys
 // through four layers of the 30B-A3B shape took 7.5 ms unsplit (2.8 ms token
 // by token), so 1.2; after 4000 keys 1.31, 1.31 and 0.77 ms.
+//
+// The matrix products give every query of a tile every V row up to the
+// largest key met, those it does not see times 0.  Where the batch wrote a V
+// value that is not finite (a.odd), 0 times it would put NaN into the tokens
+// before it: each query is then taken by a wave of its own, over the keys it
+// sees only (prompt_attn_rows).
+__device__ __forceinline__ void prompt_attn_emit(const PromptAttn &a, int HD, int64_t o, int d, float O, float L, float M)
+{
+    if (gridDim.z == 1) {
+        a.out[o * HD + d] = O / L;
+        return;
+    }
+    float *p = a.part + (o * gridDim.z + blockIdx.z) * (HD + 2);
+    p[2 + d] = O;
+    if (d == 0) p[0] = M, p[1] = L;
+}
+
+template <int HD> __device__ __forceinline__ void prompt_attn_rows(const PromptAttn &a)
+{
+    const int lane = threadIdx.x & 63, gqa = a.nh / a.nkv, kvh = blockIdx.y, r0 = blockIdx.x * 16;
+    const int r1 = min(r0 + 16, a.T * gqa), c0 = blockIdx.z * a.chunk;
+    auto row_at = [&](int key) {
+        return (((int64_t)a.page_table[key / a.page_tokens] * a.nkv + kvh) * a.page_tokens + key % a.page_tokens) * HD;
+    };
+    for (int r = r0 + (threadIdx.x >> 6); r < r1; r += PWG / 64) {
+        const int64_t oi = (int64_t)(r / gqa) * a.nh + kvh * gqa + r % gqa;
+        const int last = min(a.pos0 + r / gqa, c0 + a.chunk - 1);
+        const float *q = a.q + oi * HD;
+        float m = -INFINITY, l = 0.0f, o[HD / 64] = {};
+        for (int k0 = c0; k0 <= last; k0 += 64) {
+            const float *kp = a.kpool + row_at(min(k0 + lane, last));
+            float s = 0.0f;
+#pragma unroll 2
+            for (int d = 0; d < HD; d += 4) {
+                const f4 x = ld4(q + d), k = ld4(kp + d);
+                s += (x.x * k.x + x.y * k.y) + (x.z * k.z + x.w * k.w);
+            }
+            s = k0 + lane <= last ? s * a.scale : -INFINITY;
+            const float mn = fmaxf(m, wave_max(s)), mz = mn == -INFINITY ? 0.0f : mn;
+            const float corr = expf(m - mz), p = expf(s - mz);
+            m = mn;
+            l = l * corr + wave_sum(p);
+#pragma unroll
+            for (int i = 0; i < HD / 64; i++) o[i] *= corr;
+            for (int j = 0; j < min(64, last - k0 + 1); j++) {
+                const float *vp = a.vpool + row_at(k0 + j) + lane;
+                const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), j));
+#pragma unroll
+                for (int i = 0; i < HD / 64; i++) o[i] += pj * vp[64 * i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < HD / 64; i++) prompt_attn_emit(a, HD, oi, lane + 64 * i, o[i], l, m);
+    }
+}
+
 template <int HD> __global__ void __launch_bounds__(PWG) k_prompt_attn(PromptAttn a)
 {
     __shared__ __align__(16) Merge16<HD> s;
+    if (*a.odd) {
+        prompt_attn_rows<HD>(a);
+        return;
+    }
     const int wave = threadIdx.x >> 6, n = threadIdx.x & 15;
     const int gqa = a.nh / a.nkv, kvh = blockIdx.y, nrow = a.T * gqa, r0 = blockIdx.x * 16;
     const int row = min(r0 + n, nrow - 1);
@@ -894,20 +961,13 @@ template <int HD> __global__ void __launch_bounds__(PWG) k_prompt_attn(PromptAtt
     attn16_merge<HD>(at, s, [&](int r, int d, float O, float L, float M) {
         const int qr = r0 + r;
         if (qr >= nrow) return;
-        const int64_t o = (int64_t)(qr / gqa) * a.nh + kvh * gqa + qr % gqa;
-        if (gridDim.z == 1) {
-            a.out[o * HD + d] = O / L;
-            return;
-        }
-        float *p = a.part + (o * gridDim.z + blockIdx.z) * (HD + 2);
-        p[2 + d] = O;
-        if (d == 0) p[0] = M, p[1] = L;
+        prompt_attn_emit(a, HD, (int64_t)(qr / gqa) * a.nh + kvh * gqa + qr % gqa, d, O, L, M);
     });
 }
 
 static bool attn_ok(const PromptAttn &a)
 {
-    return a.T >= 1 && a.nkv >= 1 && a.nh >= a.nkv && a.nh % a.nkv == 0 && a.pos0 >= 0 &&
+    return a.odd && a.T >= 1 && a.nkv >= 1 && a.nh >= a.nkv && a.nh % a.nkv == 0 && a.pos0 >= 0 &&
            (a.hd == 64 || a.hd == 128 || a.hd == 256) && a.page_tokens >= A16_KB && a.page_tokens % A16_KB == 0;
 }
 

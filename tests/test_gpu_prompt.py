@@ -181,6 +181,7 @@ def test_batch_lengths(gpu, n):
     dict(n_heads=2, n_kv_heads=2, head_dim=256),
     dict(n_ff_shexp=256), dict(n_ff_shexp=96, exp_type=(Q8_0, Q8_0, Q8_0)),   # shared expert
     dict(router_zipf_s=1.1),                                                  # router bias
+    dict(embd_type=0), dict(embd_type=1),                                     # f32, f16 embeddings
 ])
 def test_types_and_shapes(gpu, kw):
     check(gpu, cfg(**kw), 40)
@@ -195,6 +196,42 @@ def test_several_batches_and_pages(gpu):
 def test_host_experts(gpu, budget, arena):
     """Experts in pinned host memory, read in place by the batch."""
     check(gpu, cfg(), 40, expert_budget_mb=budget, arena=arena)
+
+
+# 16 tokens a row tile, 2 tokens a row tile, keys in several chunks
+@pytest.mark.parametrize("nh,nkv,past", [(4, 4, 0), (16, 2, 0), (4, 4, 900)])
+def test_token_without_finite_values(gpu, tmp_path, nh, nkv, past):
+    """A token whose embedding row is not finite: the rows of the tokens
+    before it are what they are token by token, its own is not finite."""
+    from styx_amd import MoeModel, gguf_io
+    c = cfg(n_heads=nh, n_kv_heads=nkv, embd_type=1, seed=31)
+    m = MoeModel.synth(gpu, c, n_ctx=32)
+    tensors = []
+    for name in m.tensor_names():
+        t, dims, data = m.export_tensor(name)
+        if name == "token_embd.weight":
+            data = data.copy()
+            data.view(np.uint16).reshape(c.n_vocab, c.n_embd)[7, 5] = 0x7C00  # inf
+        tensors.append((name, t, dims, data))
+    path = tmp_path / "m.gguf"
+    gguf_io.write(path, gguf_io.model_metadata({k: getattr(m.hp, k) for k in (
+        "n_layers", "n_embd", "n_heads", "n_kv_heads", "head_dim", "n_expert", "n_expert_used", "n_ff_exp",
+        "rms_eps", "rope_base")}), tensors)
+    m.close()
+    toks = np.arange(100, 123, dtype=np.uint32)
+    toks[12] = 7
+    a, b = (MoeModel.load(gpu, str(path), n_ctx=past + 32) for _ in range(2))
+    if past:
+        a.fill_kv(past)
+        b.fill_kv(past)
+    a.generate(toks, 1)
+    for t in toks:
+        b.forward_token(int(t), False)
+    for x, y in zip(a.read_kv(1, past, 22), b.read_kv(1, past, 22)):
+        assert np.isfinite(y[:12]).all() and rel_l2(x[:12], y[:12]) < TOL
+        assert not np.isfinite(x[12]).any() and not np.isfinite(y[12]).any()
+    a.close()
+    b.close()
 
 
 def test_prompt_after_prompt(gpu):
