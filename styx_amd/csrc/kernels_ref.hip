@@ -154,12 +154,15 @@ template <int HD> __global__ void __launch_bounds__(256) kr_attn16(AttnRef a)
     const uint32_t kvh = blockIdx.y / a.tiles, h0 = kvh * a.gqa + blockIdx.y % a.tiles * 16;
     const uint32_t nrow = min(min(a.gqa - blockIdx.y % a.tiles * 16, 16u), a.nh - min(h0, a.nh));
     if (nrow == 0) return;
-    const uint32_t c0 = blockIdx.x * a.chunk, c1 = min(a.n_t, c0 + a.chunk);
+    const uint32_t c0 = blockIdx.x * a.chunk, nk = min(a.n_t - c0, a.chunk);
     Attn16<HD> at;
     at.init(a.Q + (int64_t)(h0 + min((uint32_t)(threadIdx.x & 15), nrow - 1)) * HD);
-    for (uint32_t k0 = c0 + (threadIdx.x >> 6) * A16_KB; k0 < c1; k0 += 4 * A16_KB) {
-        const int64_t base = (int64_t)k0 * a.kv_dim + (int64_t)kvh * HD;
-        const int left = (int)min(c1 - k0, (uint32_t)A16_KB);
+    // keys left to this wave, counted down: n_t may be anything up to 2^32 - 1
+    // (rows that overlap, kv_dim 0), past which a key position would wrap
+    const uint32_t k0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * A16_KB;
+    int64_t base = (int64_t)(c0 + k0) * a.kv_dim + (int64_t)kvh * HD;
+    for (uint32_t rem = nk - min(nk, k0); rem > 0; rem -= min(rem, 4u * A16_KB), base += 4 * A16_KB * (int64_t)a.kv_dim) {
+        const int left = (int)min(rem, (uint32_t)A16_KB);
         at.block(a.K + base, a.V + base, a.kv_dim, left - 1, left, a.scale);
     }
     attn16_merge<HD>(at, s, [&](int r, int d, float O, float L, float M) {
@@ -167,10 +170,10 @@ template <int HD> __global__ void __launch_bounds__(256) kr_attn16(AttnRef a)
         const int64_t h = h0 + r;
         // the last block's missing keys are 0 times its last row: where that
         // holds an infinity, the keys' own sum
-        if (O != O && isinf(a.V[(int64_t)(c1 - 1) * a.kv_dim + (int64_t)kvh * HD + d])) {
+        if (O != O && isinf(a.V[(int64_t)(c0 + nk - 1) * a.kv_dim + (int64_t)kvh * HD + d])) {
             O = 0.0f;
-            for (uint32_t k = c0; k < c1; k++) {
-                const int64_t row = (int64_t)k * a.kv_dim + (int64_t)kvh * HD;
+            for (uint32_t k = 0; k < nk; k++) {
+                const int64_t row = (int64_t)(c0 + k) * a.kv_dim + (int64_t)kvh * HD;
                 float x = 0.0f;
 #pragma unroll 4
                 for (int i = 0; i < HD; i++) x += a.Q[h * HD + i] * a.K[row + i];
@@ -230,7 +233,7 @@ static hipError_t attn_go(hipStream_t st, AttnRef a, uint32_t hd, const RefScrat
     const uint64_t ny = (uint64_t)((a.nh + a.gqa - 1) / a.gqa) * a.tiles;
     if (ny > 65535) return hipErrorNotSupported;
     a.chunk = attn_chunk_keys(a.n_t, ny, a.nh, hd, s && s->p ? s->floats : 0);
-    const uint32_t chunks = (a.n_t + a.chunk - 1) / a.chunk;
+    const uint32_t chunks = (uint32_t)(((uint64_t)a.n_t + a.chunk - 1) / a.chunk);
     a.part = chunks > 1 ? s->p : nullptr;
     const dim3 grid(chunks, (unsigned)ny);
     if (hd == 64)

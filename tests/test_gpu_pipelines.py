@@ -201,6 +201,23 @@ def test_attn_decode_shapes(gpu, n_t, hd, nh, gqa, pad):
     assert (got[nh * hd:] == 3.0).all()
 
 
+def test_attn_decode_overlapping_rows_and_the_largest_context(gpu):
+    """kv_dim 0: every key is the same row, whatever n_t says, up to 2^32 - 1
+    (key positions in 64 bits; counted in 32 the last blocks never ended)."""
+    hd, nh = 64, 4
+    rng = np.random.default_rng(0)
+    q, K, V = (rng.standard_normal(n).astype(np.float32) for n in (nh * hd, hd, hd))
+    for n_t in (5, 300, 70001, 2 ** 32 - 1):
+        bo = gpu.zeros(nh * hd * 4)
+        run(gpu, "attn_decode_f32", [f32buf(gpu, q), f32buf(gpu, K), f32buf(gpu, V), bo],
+            struct.pack("<4If", n_t, hd, 0, nh, 0.125), (nh, 1, 1))
+        # every key adds the same value, so roundings do not average: a wave
+        # adds up its blocks in turn (at most 512 chunks, 4 waves, 32 keys),
+        # then come 32 keys within a block, 4 waves and the chunks
+        adds = n_t / (512 * 4 * 32) + 32 + 4 + 512
+        assert rel_l2(bo.download(np.float32).reshape(nh, hd), np.tile(V, (nh, 1))) < adds * 2.0 ** -24, n_t
+
+
 # contexts that end inside a key block, one and several chunks
 @pytest.mark.parametrize("n_t,hd,gqa", [(1, 64, 1), (31, 128, 4), (32, 128, 4), (33, 256, 2), (257, 64, 8),
                                         (600, 128, 4)])
