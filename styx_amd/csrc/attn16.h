@@ -13,6 +13,7 @@
 #include <algorithm>
 
 #include "qdot.h"
+#include "refk.h"
 
 namespace styx {
 
@@ -181,7 +182,7 @@ __device__ __forceinline__ void attn16_merge(const Attn16<HD> &a, Merge16<HD> &s
 // partials [rows][chunks][hd + 2] fit `floats`.
 inline uint32_t attn_chunk_keys(uint64_t n_t, uint64_t groups, uint64_t rows, uint64_t hd, uint64_t floats)
 {
-    if (n_t <= 256) return (uint32_t)n_t;
+    if (n_t <= REF_ATTN_WHOLE) return (uint32_t)n_t;
     const uint64_t most = std::min<uint64_t>(512 / std::min<uint64_t>(groups, 512), floats / (rows * (hd + 2)));
     if (most < 2) return (uint32_t)n_t;
     return (uint32_t)std::min<uint64_t>(n_t, (n_t + 128 * most - 1) / (128 * most) * 128);

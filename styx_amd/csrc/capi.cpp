@@ -59,6 +59,8 @@ static void gpu_destroy(styx_gpu *g)
     if (g->xq_scratch) hipFree(g->xq_scratch);
     if (g->partial_scratch) hipFree(g->partial_scratch);
     if (g->ref_part) hipFree(g->ref_part);
+    for (float *p : g->ref_spare)
+        if (p) hipFree(p);
     if (g->fused_scalars) hipFree(g->fused_scalars);
     if (g->fused_pt) hipFree(g->fused_pt);
     delete g;
@@ -114,7 +116,6 @@ int styx_gpu_new(int device, styx_gpu **out)
     if (e != hipSuccess) {
         if (g->xq_scratch) hipFree(g->xq_scratch);
         if (g->partial_scratch) hipFree(g->partial_scratch);
-    if (g->ref_part) hipFree(g->ref_part);
         if (g->fused_scalars) hipFree(g->fused_scalars);
         if (g->fused_pt) hipFree(g->fused_pt);
         hipStreamDestroy(g->stream);

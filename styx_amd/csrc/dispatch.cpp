@@ -101,11 +101,15 @@ struct styx_timeline {
 namespace {
 
 // Attention partials for work on b's stream: the batch's own when it has a
-// stream of its own, else the gpu's (its caller holds ref_mu).  Without
-// memory for them contexts are not split.
+// stream of its own (kept until it is freed, then for the next batch), else
+// the gpu's.  The caller holds ref_mu.  Without memory for them contexts are
+// not split.
 RefScratch ref_scratch(styx_batch *b)
 {
     float *&p = b->own ? b->part : b->gpu->ref_part;
+    if (!p && b->own)
+        for (float *&s : b->gpu->ref_spare)
+            if (s && !p) std::swap(p, s);
     if (!p && hipMalloc((void **)&p, REF_SCRATCH_FLOATS * sizeof(float)) != hipSuccess) {
         (void)hipGetLastError();
         p = nullptr;
@@ -119,9 +123,12 @@ int run_cmds(styx_batch *b, hipStream_t st)
     for (auto &c : b->cmds) {
         std::unique_lock<std::mutex> lock;
         RefScratch scratch{};
-        if (c.k->kid == RK_ATTN) {
-            if (!b->own) lock = std::unique_lock<std::mutex>(b->gpu->ref_mu);
+        uint32_t n_t = 0;
+        if (c.k->kid == RK_ATTN) std::memcpy(&n_t, c.push.data(), 4);
+        if (n_t > REF_ATTN_WHOLE) {
+            lock = std::unique_lock<std::mutex>(b->gpu->ref_mu);
             scratch = ref_scratch(b);
+            if (b->own) lock.unlock();
         }
         const uint32_t *spec = c.k->spec.empty() ? nullptr : c.k->spec.data();
         hipError_t e = c.k->kid >= RK_F_ROUTER_TOPK
@@ -252,6 +259,14 @@ void styx_batch_free(styx_batch *b)
         hipStreamSynchronize(b->own);
         hipEventDestroy(b->done);
         hipStreamDestroy(b->own);
+        if (b->part) {
+            std::lock_guard<std::mutex> lock(g->ref_mu);
+            for (float *&s : g->ref_spare)
+                if (!s) {
+                    std::swap(s, b->part);
+                    break;
+                }
+        }
         if (b->part) hipFree(b->part);
     }
     delete b;

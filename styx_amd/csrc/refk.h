@@ -36,6 +36,7 @@ struct RefScratch {
     uint64_t floats;
 };
 constexpr uint64_t REF_SCRATCH_FLOATS = 2u * 1024u * 1024u;
+constexpr uint32_t REF_ATTN_WHOLE = 256;  // contexts of up to these keys are not split
 
 // Launch reference kernel `kid` with resolved binding pointers and the bytes
 // each binding makes visible, the raw push-constant block, the reference

@@ -38,10 +38,14 @@ struct styx_gpu {
     static constexpr int FUSED_PT_MAX = 65536;
     uint32_t *fused_pt = nullptr;
     // Attention partials of batches on `stream` (refk.h RefScratch), made at
-    // the first one and kept; ref_mu is held over a dispatch's launches, so
-    // that batches of several threads do not come between a launch that
-    // writes the partials and the one that reads them.
+    // the first split context and kept; ref_mu is held over a dispatch's
+    // launches, so that batches of several threads do not come between a
+    // launch that writes the partials and the one that reads them.
     float *ref_part = nullptr;
+    // Partials of freed async batches for the next ones (under ref_mu too):
+    // freeing them would wait for every stream of the device.
+    static constexpr int REF_SPARE = 4;
+    float *ref_spare[REF_SPARE] = {};
     std::mutex ref_mu;
 };
 

@@ -268,6 +268,36 @@ def test_attn_in_async_and_plain_batches(gpu):
         o.free()
 
 
+def test_freeing_an_async_batch_waits_for_its_own_stream_only(gpu):
+    """A batch that ran attention is freed while another batch's work runs on
+    (freeing its partials to the device would wait for that)."""
+    import time
+    from styx_amd.runtime import Batch, Kernel, Timeline
+    rows, cols, n_t, hd = 16384, 8192, 2000, 128
+    a = [gpu.zeros(rows * cols // 32 * 34), f32buf(gpu, np.ones(cols)), gpu.zeros(rows * 4), gpu.zeros(16),
+         gpu.zeros(16)]
+    mv, at, t = Kernel(gpu, "mul_mat_vec_q8_0_f32_f32", [(1, 1)]), Kernel(gpu, "attn_decode_f32", []), Timeline(gpu)
+    push = struct.pack("<13I", cols, cols // 32, cols, rows, rows * cols, cols, rows, 0, 0, 1, 1, 1, 1)
+    kv = [gpu.zeros(hd * 4), gpu.zeros(n_t * hd * 4), gpu.zeros(n_t * hd * 4), gpu.zeros(hd * 4)]
+    work, b = Batch(gpu, is_async=True), Batch(gpu, is_async=True)
+    b.begin()
+    b.dispatch(at, kv, struct.pack("<4If", n_t, hd, hd, 1, 0.1), (1, 1, 1))
+    b.submit_async(t, 1)
+    b.wait_idle()
+    work.begin()
+    for _ in range(600):  # about 45 ms
+        work.dispatch(mv, a, push, (rows, 1, 1))
+    work.submit_async(t, 2)
+    t0 = time.perf_counter()
+    b.free()
+    t1 = time.perf_counter()
+    work.wait_idle()
+    t2 = time.perf_counter()
+    for o in (work, mv, at, t):
+        o.free()
+    assert t1 - t0 < 0.5 * (t2 - t1), (t1 - t0, t2 - t1)
+
+
 # op matvec: limbs built by the workgroups (up to 2048 columns, or few rows)
 # or by a launch in front (long rows of many rows, outputs over the input)
 @pytest.mark.parametrize("t,rows,cols", [(8, 40, 32), (8, 33, 2048), (8, 16, 2112), (12, 64, 4096),
