@@ -57,7 +57,6 @@ def check(gpu, c, n_prompt, oracle=True, n_ctx=None, **opts):
             assert rel_l2(x, y) < TOL, layer
             rows = np.linalg.norm(x - y, axis=1) / np.linalg.norm(y, axis=1)
             assert rows.max() < TOL, (layer, int(rows.argmax()))
-    assert (a.last_expert_ids().shape == b.last_expert_ids().shape)
     la = a.forward_token(int(toks[1]))
     b.forward_token(int(toks[0]))
     lb = b.forward_token(int(toks[1]))
@@ -65,8 +64,10 @@ def check(gpu, c, n_prompt, oracle=True, n_ctx=None, **opts):
     if oracle:
         orc = oracle_from_model(b, n_ctx)
         for pos, t in enumerate([*prompt.tolist(), *toks.tolist()]):
-            ol, *_ = orc.forward(pos, int(t))
+            ol, _, _, margins = orc.forward(pos, int(t))
         assert rel_l2(la, ol) < 1e-4
+        clear = np.asarray(margins) > 1e-4  # (layers that route without a doubt)
+        assert np.array_equal(a.last_expert_ids()[clear], b.last_expert_ids()[clear])
     a.close()
     b.close()
 
@@ -194,8 +195,32 @@ def test_several_batches_and_pages(gpu):
 
 @pytest.mark.parametrize("budget,arena", [(0, True), (1, False)])
 def test_host_experts(gpu, budget, arena):
-    """Experts in pinned host memory, read in place by the batch."""
+    """Experts in pinned host memory: every slab that the batch meets passes
+    through its 64 MiB staging buffer."""
     check(gpu, cfg(), 40, expert_budget_mb=budget, arena=arena)
+
+
+@pytest.mark.parametrize("kw", [
+    # about 54 experts met, 40 slabs of 1.7 MB to the buffer: the others are read in place
+    dict(n_embd=2048, n_ff_exp=768, n_expert=64, n_expert_used=8, exp_type=(Q8_0, Q8_0, Q8_0)),
+    # slabs of 36 MB, one to the buffer, and of 71 MB, none
+    dict(n_embd=8192, n_ff_exp=8192, n_expert=16, n_expert_used=2, exp_type=(Q4_K, Q4_K, Q8_0)),
+])
+def test_host_experts_past_the_staging_buffer(gpu, kw):
+    from styx_amd import MoeModel
+    m = MoeModel.synth(gpu, cfg(**kw), n_ctx=64, expert_budget_mb=0)
+    toks = np.random.default_rng(2).integers(0, 1024, 41).astype(np.uint32)
+    m.generate(toks, 1)
+    batch = m.read_kv(1, 0, 40)
+    m.reset()
+    met = set()
+    for t in toks:
+        m.forward_token(int(t), False)
+        met |= set(m.last_expert_ids()[0].tolist())
+    assert len(met) > (64 << 20) // (kw["n_embd"] * kw["n_ff_exp"] // 32 * 34)
+    for x, y in zip(batch, m.read_kv(1, 0, 40)):
+        assert (np.linalg.norm(x - y, axis=1) < TOL * np.linalg.norm(y, axis=1)).all()
+    m.close()
 
 
 # 16 tokens a row tile, 2 tokens a row tile, keys in several chunks
