@@ -22,16 +22,16 @@
 // all exact in f16 (q6_K's 12-bit products with its 8-bit scale are an f16
 // plus an exact remainder).  An activation row is scaled by a power of two so
 // that its largest value lies in [2^13, 2^14) and written as three f16 pieces
-// x = p1 + p2 + p3, p1 a multiple of 16 and p2 of 2^-7: 33 bits below the
-// row's maximum.  v_mfma_f32_16x16x32_f16 forms exact products, and sums of
+// x = p1 + p2 + p3, p1 a multiple of 16, p2 and p3 each the rounding of what
+// is left: 23 bits of every value, to 39 bits below the row's maximum.  v_mfma_f32_16x16x32_f16 forms exact products, and sums of
 // integers below 2^24 are exact in its f32 accumulator, so p1's products of
 // 256 values (integers times 16) are summed without an error to speak of; the
-// products of p2 and p3 go into an accumulator of their own.  (With pieces
-// that are each the rounding of what the previous ones leave, the low bits of
-// every addition were dropped downwards by the matrix core.)  A matrix's f16
+// products of p2 and p3 go into an accumulator of their own.  (With a first
+// piece that is just x's rounding, the low bits of every addition to its sum
+// were dropped downwards by the matrix core.)  A matrix's f16
 // block factor multiplies the block's sum, and blocks are added up, in f64.
 // Layer-0 V rows against 64 bits, relative L2, here and token by token: q8_0
-// 7.1e-8, 8.6e-8; q4_K 9.8e-8, 1.02e-7; q5_K 9.8e-8, 1.06e-7; q6_K 5.9e-8,
+// 7.1e-8, 8.6e-8; q4_K 9.6e-8, 1.02e-7; q5_K 9.6e-8, 1.06e-7; q6_K 5.9e-8,
 // 9.0e-8 (2048 columns, 300 tokens).
 #include "attn16.h"
 #include "deq.h"
@@ -93,17 +93,17 @@ __device__ __forceinline__ float pack_max(float v, float *red)
     return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-// v = a + b + c: a a multiple of 16, b of 2^-7, c the rest (|v| < 2^14)
+// v = a + b + c: a a multiple of 16, b the rounding of the rest, c of that
+// rest's (|v| < 2^14)
 template <typename F> __device__ __forceinline__ void pieces3(F v, _Float16 &a, _Float16 &b, _Float16 &c)
 {
     // adding and taking off 1.5 2^p u, p the mantissa's length, rounds to a
     // multiple of u
     constexpr F mid = sizeof(F) == 4 ? (F)12582912.0 : (F)6755399441055744.0;
-    constexpr F g1 = mid * (F)16, g2 = mid * (F)0.0078125;
-    const F p1 = (v + g1) - g1, r1 = v - p1, p2 = (r1 + g2) - g2;
+    const F p1 = (v + mid * (F)16) - mid * (F)16, r1 = v - p1;
     a = (_Float16)(float)p1;
-    b = (_Float16)(float)p2;
-    c = (_Float16)(float)(r1 - p2);
+    b = (_Float16)(float)r1;
+    c = (_Float16)(float)(r1 - (F)b);
 }
 // v of the lane that the DPP control CTRL names
 template <int CTRL> __device__ __forceinline__ double dpp_d(double v)
@@ -537,15 +537,15 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
             } else {
                 // minimum terms: sum_j m_j s_j of the 8 sub-blocks, the third
                 // to first pieces of s_j in lane groups 0..2 (group 3
-                // multiplies zeros); the first two and the third summed apart,
-                // each exactly
+                // multiplies zeros); the first, exactly, and the other two
+                // summed apart
                 const uint32_t z = w[r].hd.z, hw = w[r].hd.w;
                 h2 e[4];
                 bytes_1024(z & 0x3F3F3F3Fu, e[0], e[1]);
                 bytes_1024(((hw >> 4) & 0x0F0F0F0Fu) | ((z >> 2) & 0x30303030u), e[2], e[3]);
                 const h2 off = dup_h2(-1024.0f);
                 const h8 mv = cat8(e[0] + off, e[1] + off, e[2] + off, e[3] + off);
-                const h8 mz = {}, mhi = g == 0 ? mz : mv, mlo = g == 0 ? mv : mz;
+                const h8 mz = {}, mhi = g < 2 ? mz : mv, mlo = g < 2 ? mv : mz;
                 const double d = f16f(w[r].hd.x), dm = -64.0 * f16f(w[r].hd.x >> 16);
 #pragma unroll
                 for (int t = 0; t < TT; t++) {
