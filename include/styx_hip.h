@@ -447,8 +447,10 @@ int styx_moe_forward_token(styx_moe *m, uint32_t token, float *logits);
  * prefill's logits), argmax on the device.  Prompts of more than 4 tokens
  * run in batches of up to 512, the last token by itself: the K/V rows and
  * logits of forwarding the tokens one by one, up to the rounding of f32
- * sums.  (Token by token with time_kernels, with repinning, or when the
- * batch workspace does not fit in HBM.) */
+ * sums.  (Token by token with time_kernels, with repinning, with rows --
+ * n_embd, n_head * head_dim, an FFN width -- of more than 15360 values, or
+ * when the batch workspace did not fit in HBM at the model's first such
+ * prompt.) */
 int styx_moe_generate(styx_moe *m, const uint32_t *prompt, int n_prompt, int n_predict,
                       uint32_t *out_tokens, double *prefill_s, double *decode_s);
 /* Continue greedy decoding from the current state: n_steps forward passes,

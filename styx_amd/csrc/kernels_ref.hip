@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256) kr_axpy_sig(const float *a, const float *
 // KB and a launch has few rows, so a row's time is its memory round trip:
 // every lane has its loads of a 2048-value pass (8 of the row, 8 of x) in
 // flight at once.  128 rows of 2048: 21.6 us with 32 lanes and one load at a
-// time, 4.9 so.
+// time, 2.6 so.
 __global__ void __launch_bounds__(64) kr_matvec_strided(const float *A, const float *x, float *d,
                                                         uint32_t ncols, uint32_t stride)
 {
@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(128) kr_attn_decode(const float *Q, const floa
 // round trips: a long context is cut into `chunk` keys per workgroup
 // (blockIdx.x) whose (m, l, o) go to part [head][chunks][hd + 2] and are
 // merged by kr_attn_merge.  Against one workgroup per query head and a
-// barrier tree per key: 145 keys 167 -> 8 us, 4000 keys 5360 -> 16 us
+// barrier tree per key: 145 keys 167 -> 16 us, 4000 keys 5360 -> 12 and 4 us
 // (32 heads, 4 kv heads of 128).
 struct AttnRef {
     const float *Q, *K, *V;
@@ -295,15 +295,16 @@ __global__ void __launch_bounds__(256) kr_rms_norm(const float *a, const float *
 // in registers over the rows its group visits and has the next row's loads
 // in flight over this row's products: f32 FMAs of weights dequantized one by
 // one, as the reference's.  (Factors taken out of the sums, d (s sum q x - m
-// sum x), cost a quarter of the instructions and no time, but cancel: q6_K
-// rows times activations around 1 were 5.0e-7 off 64 bits, so 1.3e-7, and an
+// sum x), save a third of the products' instructions, which shows in long
+// matrices of q6_K only, 151936 x 2048 59 us, so 73; but they cancel: q6_K
+// rows times activations around 1 were 5.0e-7 off 64 bits, so 1.0e-7, and an
 // infinite activation gave NaN where its row's sum is infinite.)
 //
 // Bound: the memory round trip at one expert's few rows, the weight stream
 // beyond.  Against one lane per block and byte loads into a dequantized
 // array in scratch memory (8 of 64 lanes busy on a 2048-column K-quant row),
-// 30B-A3B layer: gate q4_K 183 -> 8, up q5_K 178 -> 8, down q6_K 382 -> 9,
-// q q8_0 24 -> 6 us.
+// 30B-A3B layer: gate q4_K 183 -> 6, up q5_K 178 -> 6, down q6_K 382 -> 8,
+// q q8_0 24 -> 8 us.
 struct MmvRef {
     const uint8_t *A;
     const float *B;

@@ -569,10 +569,11 @@ __device__ __forceinline__ void gemm_step(const PW<T, D8> (&w)[NG], XOp xop, SOp
 // Bound: the weight stream while an expert has few tokens, the matrix cores
 // (three or four f16 products per value) beyond; 16 TT = 32 tokens keeps an
 // expert's tile near the 24 tokens an expert meets in 384-token prompts at
-// k / E = 8 / 128 and two workgroups on a CU.  At 383 tokens of the 30B-A3B
-// shape: q/k/v (5120 x 2048 q8_0) 48 us, gate (q4_K) 87, up (q5_K) 111, down
-// (q6_K) 90 us for 417 MB of slabs; a 384-token prompt through two such
-// layers took 51.7 ms token by token and takes 1.0 ms (with two generated
+// k / E = 8 / 128 and two workgroups on a CU (the second launch bound, in
+// waves per SIMD).  At 383 tokens of the 30B-A3B shape: q/k/v (5120 x 2048
+// q8_0) 49 us, o-proj (2048 x 4096) 59, gate (q4_K) 85, up (q5_K) 104, down
+// (q6_K) 100 us for 417 MB of slabs; a 384-token prompt through two such
+// layers took 50.7 ms token by token and takes 1.0 ms (with two generated
 // tokens), the batch itself 0.53 ms.
 template <int T, bool D8, int TT, int NG, int NW>
 __global__ void __launch_bounds__(64 * NW, NW / 2) k_prompt_gemm(PromptGemm a)
@@ -705,8 +706,8 @@ __global__ void __launch_bounds__(64 * NW, NW / 2) k_prompt_gemm(PromptGemm a)
 // activations straight from the L2, and the waves' sums meet in LDS.  A
 // workgroup of the kernel above walks all steps in turn, each a memory round
 // trip of about 3 us while few workgroups share a CU: q8_0 q/k/v (5120 x
-// 2048) 26 us at 9 and 19 tokens, here 15 and 23; o-proj (2048 x 4096) 48,
-// here 16 and 24; k/v (1024 x 2048) 25, here 8 and 12.  From 33 tokens on the
+// 2048) 26 us at up to 32 tokens, here 14 up to 16 and 25 above; o-proj
+// (2048 x 4096) 48, here 15 and 27.  From 33 tokens on the
 // activations' L2 traffic (every workgroup reads them all) outweighs it.
 template <int T, bool D8, int TT> __global__ void __launch_bounds__(PWG, 2) k_prompt_gemm_few(PromptGemm a)
 {

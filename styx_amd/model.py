@@ -49,9 +49,9 @@ class SynthConfig:
         return c
 
 
-# the 48-layer Qwen3-30B-A3B shape, mixed K-quant experts.
+# The 48-layer Qwen3-30B-A3B shape, mixed K-quant experts.
 CFG_30B_A3B = SynthConfig(exp_mix=True)
-# one qwen3moe layer, all q8_0 (vocab kept small: only the MoE block matters).
+# One qwen3moe layer, all q8_0 (vocab kept small: only the MoE block matters).
 CFG_LAYER_Q8 = SynthConfig(n_layers=1, n_vocab=4096)
 
 
