@@ -84,7 +84,8 @@ __global__ void __launch_bounds__(64) kr_matvec_strided(const float *A, const fl
 #pragma clang fp contract(off)
 
 // shaders/attn_decode_f32.comp:31-79 (one workgroup of 128 per query head),
-// for head dimensions without a matrix-core kernel and for empty contexts.
+// for head dimensions without a matrix-core kernel and for the shortest
+// contexts, empty ones among them.
 __global__ void __launch_bounds__(128) kr_attn_decode(const float *Q, const float *K,
                                                       const float *V, float *O, uint32_t n_t,
                                                       uint32_t hd, uint32_t kv_dim, uint32_t gqa,
@@ -679,7 +680,12 @@ hipError_t refk_launch(hipStream_t st, int kid, void *const *ptr, const uint64_t
         if (!fits(size[0], (uint64_t)gx * hd, 4) || !fits(size[1], kv_need, 4) ||
             !fits(size[2], kv_need, 4) || !fits(size[3], (uint64_t)gx * hd, 4))
             return bad;
-        if (n_t > 0 && (hd == 64 || hd == 128 || hd == 256)) {
+        // A block of 32 keys costs the matrix-core kernel the same however few
+        // it has, so up to hd / 32 keys one workgroup per head is faster.  us
+        // per head dimension, general and matrix-core kernel: 64, 2 and 3
+        // keys: 5.8 and 7.4, 6.7 and 7.0; 128, 4 and 5: 7.7 and 9.3, 8.5 and
+        // 9.0; 256, 8 and 9: 12.7 and 14.7, 13.7 and 14.4, 1: 5.6 and 14.5.
+        if (n_t > hd / 32 && (hd == 64 || hd == 128 || hd == 256)) {
             AttnRef a{};
             a.Q = (const float *)ptr[0];
             a.K = (const float *)ptr[1];

@@ -183,7 +183,9 @@ def test_matvec_strided_shapes(gpu, E, H, stride):
 @pytest.mark.parametrize("n_t,hd,nh,gqa,pad", [
     (1, 64, 4, 1, 0), (31, 128, 8, 8, 0), (33, 256, 6, 3, 0), (129, 64, 20, 20, 0), (256, 128, 32, 8, 0),
     (257, 128, 32, 8, 0), (300, 256, 16, 16, 0), (1000, 64, 7, 4, 0), (1023, 128, 10, 5, 1),
-    (9000, 64, 2, 1, 0), (700, 96, 8, 4, 0)])
+    (9000, 64, 2, 1, 0), (700, 96, 8, 4, 0),
+    # the longest contexts of the general kernel and one key more
+    (2, 64, 8, 4, 1), (3, 64, 8, 4, 1), (4, 128, 32, 8, 0), (5, 128, 32, 8, 0), (8, 256, 6, 3, 0), (9, 256, 6, 3, 0)])
 def test_attn_decode_shapes(gpu, n_t, hd, nh, gqa, pad):
     rng = np.random.default_rng(n_t + hd)
     nkv = -(-nh // gqa)
