@@ -382,11 +382,16 @@ hipError_t launch_dense_f32(hipStream_t st, int t, const uint8_t *w, int nrows, 
     // workgroups would still read x, and for long rows of many-row matrices:
     // past 2048 columns the vector is read only after the weights are issued
     // and its limbs cost the weights' registers, which a workgroup of few
-    // rows (up to 4096 rows in all) hides and one of many does not.  Limbs
-    // first -> built here: 512 x 2048 q8_0 with norm 8.0 -> 4.5 us, 151936 x
-    // 2048 q6_K 49.6 -> 45.3, 2048 x 8192 q6_K 12.3 -> 9.5; but 16384 x 8192
-    // q6_K 44.9 -> 49.7, 16384 x 6144 q4_K 23.6 -> 34.6.
-    if (overlap(x, ncols, y, nrows) || overlap(norm_w, ncols, y, nrows) || (ncols > 8 * WG && nrows > 4096)) {
+    // rows (up to 4096 rows in all) hides and one of many does not; q4_K,
+    // whose weights take the least time, hides less: up to 2048 rows past
+    // 4096 columns with a norm and 6144 without.  Limbs first -> built here,
+    // us: 512 x 2048 q8_0 with norm 8.0 -> 4.5, 151936 x 2048 q6_K 49.6 ->
+    // 45.3, 2048 x 8192 q6_K 12.1 -> 8.9, 4096 x 8192 17.6 -> 17.1, q4_K
+    // 2048 x 8192 10.4 -> 8.1; but 16384 x 8192 q6_K 44.9 -> 49.7, 16384 x
+    // 6144 q4_K 23.6 -> 34.6, q4_K with norm 4096 x 8192 13.2 -> 15.5, 2304
+    // x 5120 10.9 -> 11.8 (without 10.4 -> 10.0; 3072 x 7168 10.7 -> 11.4).
+    const int most = t == T_Q4_K && ncols > (norm_w ? 4096 : 6144) ? 2048 : 4096;
+    if (overlap(x, ncols, y, nrows) || overlap(norm_w, ncols, y, nrows) || (ncols > 8 * WG && nrows > most)) {
         hipError_t e = launch_xq(st, x, nullptr, norm_w, eps, ncols, scratch, nullptr);
         if (e != hipSuccess) return e;
         DenseSeg s{w, y, nrows};

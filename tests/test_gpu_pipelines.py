@@ -303,7 +303,8 @@ def test_freeing_an_async_batch_waits_for_its_own_stream_only(gpu):
 # op matvec: limbs built by the workgroups (up to 2048 columns, or few rows)
 # or by a launch in front (long rows of many rows, outputs over the input)
 @pytest.mark.parametrize("t,rows,cols", [(8, 40, 32), (8, 33, 2048), (8, 16, 2112), (12, 64, 4096),
-                                         (14, 4096, 3072), (14, 4098, 3072), (13, 24, 8192)])
+                                         (14, 4096, 3072), (14, 4098, 3072), (13, 24, 8192),
+                                         (12, 2048, 4352), (12, 2050, 4352), (12, 2050, 4096)])
 @pytest.mark.parametrize("norm", [False, True])
 def test_op_matvec_against_f64(gpu, t, rows, cols, norm):
     import ctypes as C
