@@ -673,8 +673,15 @@ hipError_t launch_moe_gate_up(hipStream_t st, int tg, int tu, const ExpSrc &g, c
     if (x && (route || H > XQ_MAX)) return hipErrorInvalidValue;
     // limbs built by the workgroups (30B-A3B experts: one launch less, 3.4 us)
     // unless the outputs rewrite x while other workgroups still read it, or
-    // H is past the 4096 columns this was measured to pay at
-    if (x && (H > 4096 || overlap(x, H, gu, (int64_t)2 * k * F))) {
+    // a workgroup has too many rows to hide it: more than 4096 rows past 4096
+    // columns (us, limbs first -> built: 4 x F 256 x H 8192 of q6_K 10.9 ->
+    // 7.7; limbs first there had become 11.2), or, q4_K's weights taking the
+    // least time, 100 M weights past 2048 columns (16 x F 1536 x H 3072 23.5
+    // -> 25.5, 8 x 4096 x 4096 30.5 -> 33.6; 8 x 1536 x 4096 16.8 -> 16.6).
+    const int64_t rows = (int64_t)2 * k * F;
+    const bool many = (H > 4096 && rows > 4096) ||
+                      (tg == T_Q4_K && tu == T_Q4_K && H > 2048 && rows * H > 3 << 25);
+    if (x && (many || overlap(x, H, gu, rows))) {
         hipError_t e = launch_xq(st, x, nullptr, nullptr, 0.0f, H, xq, nullptr);
         if (e != hipSuccess) return e;
         x = nullptr;

@@ -326,6 +326,36 @@ def test_op_matvec_against_f64(gpu, t, rows, cols, norm):
     assert (np.abs(by.download(np.float32, rows) - y) <= bound).all()
 
 
+# limbs built by the workgroups, or by a launch in front: past 4096 rows of
+# more than 4096 columns, and past 3 2^25 q4_K weights of more than 2048
+@pytest.mark.parametrize("t,H,F,k", [(14, 8192, 512, 4), (14, 8192, 768, 4), (8, 4352, 512, 4), (8, 4352, 544, 4),
+                                     (12, 4096, 768, 16), (12, 4096, 776, 16), (12, 2048, 1600, 16)])
+def test_op_gate_up_against_f64(gpu, t, H, F, k):
+    import ctypes as C
+    from styx_amd import _lib as L
+    from styx_amd.runtime import to_split
+    E = 2
+    be, bb = BLK[t]
+    w = [weights(t, E * F, H, t + H + i) for i in (0, 1)]
+    split = [to_split(gpu, t, gpu.from_numpy(a), F, H, E) for a in w]
+    slab = F * (H // be) * bb
+    src = [L.ExpertSrc(hot=s.ptr, hot_slab=slab) for s in split]
+    x = np.random.default_rng(H).standard_normal(H).astype(np.float32)
+    sel = np.random.default_rng(F).integers(0, E, k)
+    ids = np.full(64, -1, np.int32)
+    ids[:k] = ids[16:16 + k] = sel
+    bx, bi, gu = f32buf(gpu, x), gpu.from_numpy(ids), gpu.zeros(2 * k * F * 4)
+    L.check(gpu.lib.styx_op_moe_gate_up(gpu.h, t, t, C.byref(src[0]), C.byref(src[1]), bi.ptr, bx.ptr, gu.ptr,
+                                        H, F, k))
+    gpu.sync()
+    got = gu.download(np.float32).reshape(2, k, F)
+    for m in (0, 1):
+        y = [O.matvec_f64(t, w[m][e * slab:(e + 1) * slab], F, H, x) for e in range(E)]
+        bound = [sum_bound(t, w[m][e * slab:(e + 1) * slab], F, H, x) + 1e-6 * np.abs(y[e]).max() for e in range(E)]
+        for s, e in enumerate(sel):
+            assert (np.abs(got[m, s] - y[e]) <= bound[e]).all(), (m, s)
+
+
 def test_op_matvec_in_place(gpu):
     """y over x: the product of the old x, as with the limbs formed first."""
     import ctypes as C
